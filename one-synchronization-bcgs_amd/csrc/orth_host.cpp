@@ -37,10 +37,6 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 constexpr int kProjTargetWG = 1024;
-// Rows per CU from which a fused pass synchronizes inside its own launch
-// (2^23 rows on 256 CUs); shorter slabs end each pass with one
-// k_reduce_small launch.
-constexpr int64_t kTailMinRowsPerCU = 32768;
 
 struct DevCtx {
     std::mutex mu;
@@ -49,8 +45,10 @@ struct DevCtx {
     bool done_valid = false;
     Scratch sc;
     int ncu = 0;
-    double *Xd = nullptr;
+    double *Xd = nullptr;  // host forms: device copy of X
     size_t Xd_n = 0;
+    double *Rh = nullptr;  // host forms: pinned copy of R
+    size_t Rh_n = 0;
     int *status_h = nullptr;
     orth_status_t last = {0, 0, 0, 0, 0};
     int last_passes = 0, last_syncs = 0;
@@ -90,6 +88,17 @@ bool ensure(double *&p, size_t &cap, size_t n)
     return true;
 }
 
+bool ensure_host(double *&p, size_t &cap, size_t n)
+{
+    if (cap >= n && p) return true;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+    if (!ok(hipHostMalloc(&p, n * sizeof(double), hipHostMallocDefault))) return false;
+    cap = n;
+    return true;
+}
+
 // Grow one scratch buffer of sc to n doubles (fixed scratch: fail instead).
 bool grow(Scratch &sc, double *&p, size_t &cap, size_t n)
 {
@@ -115,7 +124,6 @@ bool ctx_init(DevCtx &c)
     if (!ok(hipMalloc(&c.sc.stash, scratch_stash_need() * sizeof(double)))) return false;
     if (!ok(hipMalloc(&c.sc.status_d, 4 * sizeof(int)))) return false;
     if (!ok(hipMalloc(&c.sc.tickets, kTailTickets * sizeof(int)))) return false;
-    c.sc.tickets_n = kTailTickets;
     if (!ok(hipHostMalloc(&c.status_h, 4 * sizeof(int), hipHostMallocDefault))) return false;
     int dev = 0;
     (void)hipGetDevice(&dev);
@@ -148,6 +156,33 @@ int block_template(int64_t s)
     if (s <= 16) return 16;
     if (s <= 32) return 32;
     return 0;
+}
+
+bool is_device_ptr(const void *p)
+{
+    if (!p) return false;
+    hipPointerAttribute_t at;
+    memset(&at, 0, sizeof(at));
+    hipError_t e = hipPointerGetAttributes(&at, p);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
+}
+
+// Can a kernel on the current device write to p?  (Pinned host memory is
+// mapped; another device's memory and pageable memory go through copies.)
+bool kernel_writable(const void *p)
+{
+    hipPointerAttribute_t at;
+    memset(&at, 0, sizeof(at));
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (at.type == hipMemoryTypeDevice) return at.device == current_device();
+    return at.type == hipMemoryTypeManaged || at.type == hipMemoryTypeHost;
 }
 
 // Records start/stop events around one launch when timing is enabled.
@@ -185,7 +220,6 @@ class Run {
         Sig_ = sc.stash;
         Om_ = Sig_ + kSlot;
         Cq_ = Om_ + kSlot;
-        Ctmp_ = Cq_ + 3 * kSlot;
     }
 
     bool prepare()
@@ -216,14 +250,16 @@ class Run {
         }
         const size_t rmax = scratch_r_need(n_);
         if (!grow(sc_, sc_.Rd, sc_.Rd_n, rmax)) return false;
-        if (!grow(sc_, sc_.Tbig, sc_.Tbig_n, scratch_tbig_need(n_))) return false;
         if (!grow(sc_, sc_.Cbuf, sc_.Cbuf_n, scratch_cbuf_need(n_))) return false;
-        if (!ok(launch_fill(sc_.Rd, rmax, st_))) return false;
-        if (!ok(launch_fill(sc_.stash, scratch_stash_need(), st_))) return false;
-        if (!ok(launch_fill_int(sc_.status_d, 4, st_))) return false;
-        if (sc_.tickets && !ok(launch_fill_int(sc_.tickets, sc_.tickets_n, st_))) return false;
         Rd_ = sc_.Rd;
-        return true;
+        SmallArgs a = sa(OP_INIT, 0, 0, 0, 0, 0, nullptr, 0);
+        a.R = Rd_;
+        a.m = (int64_t)rmax;
+        a.Sig = sc_.stash;
+        a.nslot = (int)scratch_stash_need();
+        a.status = sc_.status_d;
+        a.tickets = sc_.tickets;
+        return ok(launch_small(a, st_));
     }
 
     int64_t bw(int64_t b) const { return b == 0 ? s_ : std::min<int64_t>(s_, n_ - b * s_); }
@@ -267,14 +303,12 @@ class Run {
         a.Sig = Sig_;
         a.Om = Om_;
         a.Cq = Cq_;
-        a.Ctmp = Ctmp_;
         a.status = sc_.status_d;
-        a.Tbig = sc_.Tbig;
         a.pshift = g_pshift.load();
+        a.S = S_;
         if (fused_) {
             a.Cout = sc_.Cbuf;
             a.n1 = n1_;
-            a.S = S_;
         }
     }
 
@@ -340,11 +374,13 @@ class Run {
     // Intra-block QR of columns [col0, col0+w): shifted CholQR3; the factor
     // R3 R2 R1 goes to Rdst (ld ldRdst).  Replaces Trilinos TSQR
     // factorExplicit (SRC/orth.c:106-107 and the other TSQR call sites).
-    bool intra_qr(int64_t blk, int64_t col0, int64_t w, double *Rdst, int64_t ldRdst)
+    // flags: F_RBB to form the diagonal block of R after the last step.
+    bool intra_qr(int64_t blk, int64_t col0, int64_t w, double *Rdst, int64_t ldRdst,
+                  int flags = 0)
     {
         const int ops[3] = {OP_CQR1, OP_CQR2, OP_CQR3};
         for (int k = 0; k < 3; k++) {
-            SmallArgs a = sa(ops[k], 0, blk, 0, w, 0, nullptr, w);
+            SmallArgs a = sa(ops[k], flags, blk, col0, w, 0, nullptr, w);
             a.Rdst = Rdst;
             a.ldRdst = ldRdst;
             if (!proj(col0, w, col0, w, &a)) return false;
@@ -460,8 +496,7 @@ class Run {
             P = proj(0, c, c, wb, &q);
             if (!P) return false;
             if (!update(upd(c, wb, c, P, c, nullptr))) return false;  // :530
-            if (!intra_qr(b, c, wb, Om_, kLdT)) return false;          // :532-535
-            if (!small(sa(OP_RBB, 0, b, c, wb, 0, nullptr, 1))) return false;  // :537-541
+            if (!intra_qr(b, c, wb, Om_, kLdT, F_RBB)) return false;   // :532-541
             c += wb;
         }
         return true;
@@ -548,7 +583,7 @@ class Run {
     void set_wg_scale(double f) { wg_scale_ = std::min(1.0, std::max(f, 1e-3)); }
     // Column bound of the double-buffered s = 16 pass (0: the default).
     void set_pass16d_min_cols(int c) { minc_ = std::max(0, c); }
-    // Synchronize inside the passes (default) or in a launch after each.
+    // Allow ORTH_IN_PASS_SYNC (the reduction inside the passes).
     void set_in_pass_sync(bool on) { in_pass_sync_ = on; }
 
     // One fused pass: the pending update, then P <- A^T B (na == 0: none),
@@ -638,17 +673,17 @@ class Run {
         // registers and LDS allow.
         // The double-buffered pass with 16 waves holds a whole CU (one
         // workgroup).
-        // The pass synchronizes itself (reduction and small step in its last
-        // workgroups) when the scratch has the ticket counters and the slab
-        // is long: the tail puts device-scope cache maintenance (each
-        // workgroup's release, the last workgroups' acquires at two levels)
-        // on the critical path, 4-15 us per synchronization more than a
-        // launch boundary, which only passes of kTailMinRowsPerCU rows per CU
-        // and more hide.  Its group sums follow the partials in `part`.
-        bool tail = na > 0 && sc_.tickets && in_pass_sync_ && !getenv("ORTH_SEPARATE_REDUCE") &&
-                    !getenv("ORTH_REDUCE_LAUNCH") &&
-                    (m_ >= kTailMinRowsPerCU * (int64_t)std::max(1, c_.ncu) ||
-                     getenv("ORTH_IN_PASS_SYNC"));
+        // One k_reduce_small launch after the pass sums its partials and runs
+        // the small step.  ORTH_IN_PASS_SYNC=1 sums them in the pass's last
+        // workgroups instead and launches only the small step after it, which
+        // is slower at every size: it puts device-scope cache maintenance
+        // (each workgroup's release, the last workgroups' acquires at two
+        // levels) on the critical path.  Measured, P-1S, launch / in the
+        // pass: 203 / 231 us (4096 x 64, s = 16), 1.71 / 2.45 ms (1e5 x 200,
+        // s = 10), 144.5 / 145.2 ms (2^24 x 256, s = 16, with a 13 ms copy).
+        // The in-pass group sums follow the partials in `part`.
+        bool tail = na > 0 && sc_.tickets && in_pass_sync_ && getenv("ORTH_IN_PASS_SYNC") &&
+                    !getenv("ORTH_SEPARATE_REDUCE") && !getenv("ORTH_REDUCE_LAUNCH");
         const int per_cu = td == 16                          ? 1
                            : (ts16 > 0 || mx_ == kMxFP64) ? 2
                            : mx_                           ? 1
@@ -680,12 +715,6 @@ class Run {
             pa.tail.tickets = sc_.tickets;
             pa.tail.lvl = sc_.part + (size_t)nwg * na * nb;
             pa.tail.out = Pn;
-            if (after) {
-                pa.tail.small = 1;
-                pa.tail.sm = *after;
-                pa.tail.sm.P = Pn;
-                finish_small(pa.tail.sm);
-            }
         }
         double flops = 2.0 * m_ * na * nb, wcols = 0.0;
         for (int g = 0; g < pend_.ngrp; g++) {
@@ -711,8 +740,10 @@ class Run {
         pcur_ ^= 1;
         syncs_++;
         if (tail) {
-            if (debug_ && after) dump(pa.tail.sm);
-            return Pn;
+            if (!after) return Pn;
+            SmallArgs a = *after;
+            a.P = Pn;
+            return small(a) ? Pn : nullptr;
         }
         return sync(nwg, na, nb, Pn, after) ? Pn : nullptr;
     }
@@ -776,11 +807,12 @@ class Run {
         return pass_lds_bytes(pa) != 0;
     }
 
-    bool intra_qr_f(int64_t blk, int64_t col0, int64_t w, double *Rdst, int64_t ldRdst)
+    bool intra_qr_f(int64_t blk, int64_t col0, int64_t w, double *Rdst, int64_t ldRdst,
+                    int flags = 0)
     {
         const int ops[3] = {OP_CQR1, OP_CQR2, OP_CQR3};
         for (int k = 0; k < 3; k++) {
-            SmallArgs a = sa(ops[k], 0, blk, 0, w, 0, nullptr, w);
+            SmallArgs a = sa(ops[k], flags, blk, col0, w, 0, nullptr, w);
             a.Rdst = Rdst;
             a.ldRdst = ldRdst;
             if (!pass(col0, w, col0, w, &a)) return false;
@@ -869,8 +901,7 @@ class Run {
             if (!pass_small(0, c, c, wb, sa(OP_I2_W, 0, b, c, wb, 0, nullptr, c))) return false;
             pend_.k1 = (int)c;
             pend_group(c, wb, 0, c, nullptr);
-            if (!intra_qr_f(b, c, wb, Om_, kLdT)) return false;
-            if (!small(sa(OP_RBB, 0, b, c, wb, 0, nullptr, 1))) return false;
+            if (!intra_qr_f(b, c, wb, Om_, kLdT, F_RBB)) return false;
             c += wb;
         }
         return flush();
@@ -924,20 +955,34 @@ class Run {
         }
     }
 
-    // Copy R to the caller: for block column k only rows 0 .. end of block k.
-    bool copy_R_out(double *Rdst, int64_t ldRdst, hipMemcpyKind kind)
+    // End of the call: R to the caller's device memory (for block column k
+    // only rows 0 .. end of block k; Rdst may be null) and the first breakdown
+    // (block, pivot) to info, device or pinned host memory (may be null).
+    bool finish(double *Rdst, int64_t ldRdst, int *info)
     {
-        int64_t c = 0;
-        for (int64_t b = 0; b < N_; b++) {
-            const int64_t w = bw(b);
-            const int64_t rows = c + w;
-            if (!ok(hipMemcpy2DAsync(Rdst + c * ldRdst, ldRdst * sizeof(double),
-                                     Rd_ + c * ldR_, ldR_ * sizeof(double),
-                                     rows * sizeof(double), w, kind, st_)))
-                return false;
-            c += w;
+        SmallArgs a = sa(OP_FINISH, 0, 0, n_, s_, 0, nullptr, 0);
+        a.R = Rd_;
+        a.ldR = ldR_;
+        a.Rdst = Rdst;
+        a.ldRdst = ldRdst;
+        a.status = sc_.status_d;
+        a.info = info;
+        if (Rdst && !kernel_writable(Rdst)) {
+            a.Rdst = nullptr;
+            for (int64_t b = 0, c = 0; b < N_; c += bw(b), b++)
+                if (!ok(hipMemcpy2DAsync(Rdst + c * ldRdst, ldRdst * sizeof(double),
+                                         Rd_ + c * ldR_, ldR_ * sizeof(double),
+                                         (c + bw(b)) * sizeof(double), bw(b), hipMemcpyDefault,
+                                         st_)))
+                    return false;
         }
-        return true;
+        if (info && !kernel_writable(info)) {
+            a.info = nullptr;
+            if (!ok(hipMemcpyAsync(info, sc_.status_d, 2 * sizeof(int), hipMemcpyDefault, st_)))
+                return false;
+        }
+        if (!a.Rdst && !a.info) return true;
+        return ok(launch_small(a, st_));
     }
 
     int passes_ = 0, syncs_ = 0;
@@ -959,7 +1004,7 @@ class Run {
     void dump(const SmallArgs &a)
     {
         (void)hipStreamSynchronize(st_);
-        std::vector<double> h(6 * kSlot);
+        std::vector<double> h(5 * kSlot);
         (void)hipMemcpy(h.data(), sc_.stash, h.size() * sizeof(double), hipMemcpyDeviceToHost);
         int stat[4];
         (void)hipMemcpy(stat, sc_.status_d, sizeof(stat), hipMemcpyDeviceToHost);
@@ -973,8 +1018,8 @@ class Run {
                 for (int j = 0; j < 4 && j < a.wb; j++) fprintf(stderr, " %.6e", p[i + j * a.na]);
             fprintf(stderr, "\n");
         }
-        const char *names[6] = {"Sig", "Om", "Cq0", "Cq1", "Cq2", "Ctmp"};
-        for (int k = 0; k < 6; k++) {
+        const char *names[5] = {"Sig", "Om", "Cq0", "Cq1", "Cq2"};
+        for (int k = 0; k < 5; k++) {
             fprintf(stderr, "  %s diag:", names[k]);
             for (int i = 0; i < 4; i++) fprintf(stderr, " %.6e", h[k * kSlot + i * (kLdT + 1)]);
             fprintf(stderr, "\n");
@@ -992,22 +1037,9 @@ class Run {
     int64_t N_ = 1;
     double *Rd_ = nullptr;
     int64_t ldR_ = 0;
-    double *Sig_, *Om_, *Cq_, *Ctmp_;
+    double *Sig_, *Om_, *Cq_;
     int pcur_ = 0;
 };
-
-bool is_device_ptr(const void *p)
-{
-    if (!p) return false;
-    hipPointerAttribute_t at;
-    memset(&at, 0, sizeof(at));
-    hipError_t e = hipPointerGetAttributes(&at, p);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
-}
 
 bool shape_ok(int64_t m, int64_t n, int64_t s, int64_t ldX, int64_t ldR)
 {
@@ -1015,10 +1047,10 @@ bool shape_ok(int64_t m, int64_t n, int64_t s, int64_t ldX, int64_t ldR)
            n <= 4096;
 }
 
-// Enqueue one variant on device data.  Rdev_out receives R (device or host
-// memory, per kind).  Returns 0 or 2.
+// Enqueue one variant on device data.  Rout (device memory; null: R stays in
+// the scratch) receives R.  Returns 0 or 2.
 int run_device(DevCtx &c, int variant, int64_t m, int64_t n, int64_t s, double *dX,
-               int64_t ldX, double *Rout, int64_t ldR, hipMemcpyKind rkind, hipStream_t st,
+               int64_t ldX, double *Rout, int64_t ldR, hipStream_t st,
                int mx = 0, const float *x32 = nullptr, int64_t ldx32 = 0)
 {
     if (c.done_valid && !ok(hipStreamWaitEvent(st, c.done, 0))) return 2;
@@ -1026,10 +1058,7 @@ int run_device(DevCtx &c, int variant, int64_t m, int64_t n, int64_t s, double *
     if (mx) r.set_mixed(mx, x32, ldx32);
     if (!r.prepare()) return 2;
     if (!r.run(variant)) return 2;
-    if (!r.copy_R_out(Rout, ldR, rkind)) return 2;
-    if (!ok(hipMemcpyAsync(c.status_h, c.sc.status_d, 4 * sizeof(int), hipMemcpyDeviceToHost,
-                            st)))
-        return 2;
+    if (!r.finish(Rout, ldR, c.status_h)) return 2;
     if (!ok(hipEventRecord(c.done, st))) return 2;
     c.done_valid = true;
     c.last_passes = r.passes_;
@@ -1076,15 +1105,25 @@ int dropin(int variant, int m, int n, int s, double *X, int ldX, double *R, int 
                                  (size_t)m * sizeof(double), n, hipMemcpyHostToDevice, st)))
             return 2;
     }
-    int rc = run_device(c, variant, m, n, s, dX, ldd, R, ldR,
-                        rdev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st);
+    int rc = run_device(c, variant, m, n, s, dX, ldd, rdev ? R : nullptr, ldR, st);
     if (rc != 0) return rc;
+    if (!rdev) {
+        // R as a whole to pinned memory; the rows the caller gets from there.
+        if (!ensure_host(c.Rh, c.Rh_n, (size_t)n * n)) return 2;
+        if (!ok(hipMemcpyAsync(c.Rh, c.sc.Rd, (size_t)n * n * sizeof(double),
+                               hipMemcpyDeviceToHost, st)))
+            return 2;
+    }
     if (!xdev) {
         if (!ok(hipMemcpy2DAsync(X, (size_t)ldX * sizeof(double), dX, (size_t)ldd * sizeof(double),
                                  (size_t)m * sizeof(double), n, hipMemcpyDeviceToHost, st)))
             return 2;
     }
     if (!ok(hipStreamSynchronize(st))) return 2;
+    if (!rdev)
+        for (int64_t j = 0; j < n; j++)
+            memcpy(R + j * ldR, c.Rh + j * n,
+                   (size_t)std::min<int64_t>(n, (j / s + 1) * s) * sizeof(double));
     fill_status(c);
     return 0;
 }
@@ -1179,7 +1218,7 @@ std::vector<int64_t> shape_sig(const BatchArgs &a)
 }
 
 // Graph nodes of one instance: per synchronization a pass, a reduction and
-// a small step; the fills, the R copies and the status copy.
+// a small step; the start and the end of the call (and up to N copies of R).
 int64_t inst_nodes(int variant, int64_t n, int64_t s)
 {
     const int64_t N = 1 + (n - s + s - 1) / s;
@@ -1279,7 +1318,6 @@ bool batch_reserve(BatchCtx &b, const BatchArgs &a, int streams)
         }
         const size_t partmax = (size_t)kProjTargetWG * (nmax + 3 * kMaxS) * (3 * kMaxS);
         if (!grow(sc, sc.part, sc.part_n, partmax) || !grow(sc, sc.Rd, sc.Rd_n, scratch_r_need(nmax)) ||
-            !grow(sc, sc.Tbig, sc.Tbig_n, scratch_tbig_need(nmax)) ||
             !grow(sc, sc.Cbuf, sc.Cbuf_n, scratch_cbuf_need(nmax)))
             return false;
     }
@@ -1313,17 +1351,13 @@ bool batch_enqueue(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg,
             Run r(b.slot[k], b.slot[k].sc, a.m[i], a.n[i], a.s[i], a.X[i], a.ldX[i], st);
             r.set_wg_scale(cfg.wg_scale);
             r.set_pass16d_min_cols(cfg.minc);
-            // Concurrent instances synchronize in a launch after each pass:
-            // inside the passes, every workgroup's device-scope release and
-            // the last workgroups' acquires reach into the L2 the other
-            // streams' instances are using (the 512-instance batch ran 8 %
-            // (P-1S) and 21 % (BCGSI+) slower that way).
+            // Concurrent instances always reduce in a launch after each
+            // pass: inside the passes, the last workgroups' acquires reach
+            // into the L2 the other streams' instances are using.
             r.set_in_pass_sync(false);
             if (a.mx) r.set_mixed(a.mx, a.X32[i], a.ldX32[i]);
             good = r.prepare() && r.run(a.variant) &&
-                   r.copy_R_out(a.R[i], a.ldR[i], hipMemcpyDeviceToDevice) &&
-                   ok(hipMemcpyAsync(b.info_d + 2 * i, b.slot[k].sc.status_d, 2 * sizeof(int),
-                                     hipMemcpyDeviceToDevice, st));
+                   r.finish(a.R[i], a.ldR[i], b.info_d + 2 * i);
             if (!good) break;
         }
     }
@@ -1727,9 +1761,8 @@ int batched_entry(const BatchArgs &a, int *info, void *stream, int tune, int *cf
 
 size_t scratch_p_need(int64_t n) { return (size_t)(n + 3 * kMaxS) * (4 * kMaxS) + 64; }
 size_t scratch_r_need(int64_t n) { return (size_t)n * (n + kMaxS) + 64; }
-size_t scratch_tbig_need(int64_t n) { return (size_t)(n + kMaxS) * kMaxS; }
 size_t scratch_cbuf_need(int64_t n) { return (size_t)(n + 2 * kMaxS) * 2 * kMaxS; }
-size_t scratch_stash_need() { return 6 * (size_t)kSlot; }
+size_t scratch_stash_need() { return 5 * (size_t)kSlot; }
 
 int run_on_fixed_scratch(int variant, int64_t m, int64_t n, int64_t s, double *dX, int64_t ldX,
                          double *dR, int64_t ldR, int *dInfo, Scratch &sc, int ncu, void *stream)
@@ -1742,12 +1775,7 @@ int run_on_fixed_scratch(int variant, int64_t m, int64_t n, int64_t s, double *d
     c.ncu = ncu;
     hipStream_t st = (hipStream_t)stream;
     Run r(c, sc, m, n, s, dX, ldX, st);
-    if (!r.prepare() || !r.run(variant) || !r.copy_R_out(dR, ldR, hipMemcpyDeviceToDevice))
-        return 2;
-    if (dInfo && !ok(hipMemcpyAsync(dInfo, sc.status_d, 2 * sizeof(int), hipMemcpyDeviceToDevice,
-                                    st)))
-        return 2;
-    return 0;
+    return r.prepare() && r.run(variant) && r.finish(dR, ldR, dInfo) ? 0 : 2;
 }
 
 }  // namespace orth
@@ -1829,11 +1857,10 @@ int orth_bcgs_mixed_device(int variant, int precision, int64_t m, int64_t n, int
         // call, which may still be writing there.
         if (c.done_valid && !ok(hipStreamWaitEvent((hipStream_t)stream, c.done, 0))) return 2;
         if (!ok(launch_widen(dX32, ldX32, dQ, ldQ, m, n, (hipStream_t)stream))) return 2;
-        return run_device(c, variant, m, n, s, dQ, ldQ, dR, ldR, hipMemcpyDeviceToDevice,
-                          (hipStream_t)stream);
+        return run_device(c, variant, m, n, s, dQ, ldQ, dR, ldR, (hipStream_t)stream);
     }
-    return run_device(c, variant, m, n, s, dQ, ldQ, dR, ldR, hipMemcpyDeviceToDevice,
-                      (hipStream_t)stream, mx, dX32, ldX32);
+    return run_device(c, variant, m, n, s, dQ, ldQ, dR, ldR, (hipStream_t)stream, mx, dX32,
+                      ldX32);
 }
 
 int orth_bcgs_batched_device(int variant, int count, const int64_t *m, const int64_t *n,
@@ -1894,8 +1921,7 @@ int orth_bcgs_device(int variant, int64_t m, int64_t n, int64_t s, double *dX, i
     DevCtx &c = g_ctx[dev];
     std::lock_guard<std::mutex> lk(c.mu);
     if (!ctx_init(c)) return 2;
-    return run_device(c, variant, m, n, s, dX, ldX, dR, ldR, hipMemcpyDeviceToDevice,
-                      (hipStream_t)stream);
+    return run_device(c, variant, m, n, s, dX, ldX, dR, ldR, (hipStream_t)stream);
 }
 
 int orth_gram_device(int64_t m, const double *dX, int64_t ldX, int64_t a0, int64_t na,
@@ -2118,13 +2144,15 @@ int orth_release(void)
     std::lock_guard<std::mutex> lk(c.mu);
     if (c.done_valid) (void)hipEventSynchronize(c.done);
     auto free_scratch = [](DevCtx &x) {
-        double **bufs[] = {&x.sc.part, &x.sc.P[0], &x.sc.P[1], &x.sc.Rd, &x.sc.Tbig, &x.sc.Cbuf,
-                           &x.Xd};
+        double **bufs[] = {&x.sc.part, &x.sc.P[0], &x.sc.P[1], &x.sc.Rd, &x.sc.Cbuf, &x.Xd};
         for (double **b : bufs) {
             if (*b) (void)hipFree(*b);
             *b = nullptr;
         }
-        x.sc.part_n = x.sc.P_n = x.sc.Rd_n = x.sc.Tbig_n = x.sc.Cbuf_n = x.Xd_n = 0;
+        if (x.Rh) (void)hipHostFree(x.Rh);
+        x.Rh = nullptr;
+        x.Rh_n = 0;
+        x.sc.part_n = x.sc.P_n = x.sc.Rd_n = x.sc.Cbuf_n = x.Xd_n = 0;
     };
     free_scratch(c);
     // The batched form's captured graphs and per-stream scratch (the batch

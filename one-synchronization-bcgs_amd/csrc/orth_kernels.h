@@ -43,15 +43,17 @@ enum SmallOp {
     OP_PIPI2 = 4,       // PIPI second pass: Omega, R(0:c,b) += Y Sigma, R_bb
     OP_PLAIN_S = 5,     // R(0:c,b) = S (unnormalized first pass)
     OP_I2_W = 6,        // BCGSI+: R(0:c,b) += W Sigma
-    OP_RBB = 7,         // R_bb = Omega Sigma
     OP_CQR1 = 8,        // shifted CholQR step 1
     OP_CQR2 = 9,        // CholQR step 2
-    OP_CQR3 = 10        // CholQR step 3, writes R3 R2 R1
+    OP_CQR3 = 10,       // CholQR step 3, writes R3 R2 R1
+    OP_INIT = 11,       // start of a call: zero R, the factor slots, status, tickets
+    OP_FINISH = 12      // end of a call: R to the caller, the status to `info`
 };
 enum SmallFlag {
     F_PYTH_NEXT = 1,  // next block's Sigma from the Pythagorean Gram (P1s)
     F_1S = 2,         // R(0:c,b) = S + Y and R_bb = Omega (BCGSI+A-1S)
-    F_SEQ = 4         // emit the next pass for sequential mode (no folding)
+    F_SEQ = 4,        // emit the next pass for sequential mode (no folding)
+    F_RBB = 8         // OP_CQR3: also R_bb = (R3 R2 R1) Sigma, the diagonal block of R
 };
 
 struct SmallArgs {
@@ -66,8 +68,7 @@ struct SmallArgs {
     double *P;
     double *R;
     int64_t ldR;
-    double *Sig, *Om, *Cq, *Ctmp;  // factor slots (kSlot apart; Cq holds 3)
-    double *Tbig;                  // (n + kMaxS) x kMaxS scratch
+    double *Sig, *Om, *Cq;  // factor slots (kSlot apart; Cq holds 3)
     double *Rdst;
     int64_t ldRdst;
     int *status;  // [0] = first breakdown block (1-based), [1] = pivot
@@ -79,6 +80,14 @@ struct SmallArgs {
     // Pythagorean Cholesky steps factor G - S^T S + pshift * u * tr(G) * I
     // (u = 2^-53, G the Gram before the subtraction); 0 = no shift.
     double pshift;
+    // OP_INIT: m doubles of R, nslot doubles at Sig, status (4 ints) and
+    // kTailTickets ints of tickets (may be null) are zeroed.
+    // OP_FINISH: Rdst (ld ldRdst; may be null) receives, for every block column
+    // of width wb (the last one ragged) of the c x c matrix R, the rows down
+    // to the block's end; info (2 ints, may be null) receives status.
+    int nslot;
+    int *tickets;
+    int *info;
 };
 
 hipError_t launch_update(int S, double *X, int64_t ldX, int64_t m,
@@ -98,23 +107,21 @@ inline int tail_group(int nwg)
     return g * kTailMaxGroups < nwg ? (nwg + kTailMaxGroups - 1) / kTailMaxGroups : g;
 }
 
-// The synchronization at the end of a fused pass (the reference's
-// MPI_Allreduce and the small step after it, SRC/orth.c:114, :133, :188,
-// :197), run inside the pass launch by tickets, without waiting: the last
-// workgroup of each group to finish sums that group's partials into lvl, the
-// last of those sums the group sums into out and runs the small step.  The
-// counters are set back to zero by the workgroups that read them last.
+// The reduction at the end of a fused pass (the reference's MPI_Allreduce,
+// SRC/orth.c:114, :133, :188, :197), run inside the pass launch by tickets,
+// without waiting: the last workgroup of each group to finish sums that
+// group's partials into lvl, the last of those sums the group sums into out.
+// The counters are set back to zero by the workgroups that read them last.
 struct TailArgs {
-    int small;     // 1: after the sum, run `sm` (sm.P = out) in the last workgroup
     int nwg;       // workgroups of the pass
     int grp;       // tail_group(nwg)
-    int pad;
     int *tickets;  // [0, kTailMaxGroups) group counters, [kTailTop] the top counter
     double *lvl;   // group sums: ceil(nwg / grp) x (na nb) doubles
     double *out;   // the sum, na x nb, ld na
-    SmallArgs sm;
 };
 constexpr int kTailTop = kTailMaxGroups;
+// Ints reserved for the ticket counters (zero between launches).
+constexpr int kTailTickets = 64;
 
 // Projection partials: part[x][i + j*na] = sum over the rows of workgroup x
 // of A(:, i) * B(:, j), A = columns [a0, a0+na), B = columns [b0, b0+nb).
@@ -134,6 +141,8 @@ hipError_t launch_proj(const ProjPlan &pl, const double *X, int64_t ldX,
 hipError_t launch_reduce(const double *part, int nwg, int64_t na, int64_t nb,
                          double *out, int64_t ldo, hipStream_t st);
 
+// One small step on its own (a kernel over the device for OP_INIT and
+// OP_FINISH, one workgroup otherwise).
 hipError_t launch_small(const SmallArgs &a, hipStream_t st);
 
 // The synchronization of a pass in one launch (the reference's
@@ -169,7 +178,7 @@ struct PassArgs {
     double *X;
     int64_t ldX;
     int64_t m;
-    // 1: the pass synchronizes itself (tail below).  Beside the fields every
+    // 1: the pass reduces its own partials (tail below).  Beside the fields every
     // workgroup reads at its start, so that the check at its end finds the
     // line cached.
     int tail_on;
@@ -193,11 +202,6 @@ struct PassArgs {
     int lpb;
     TailArgs tail;
 };
-
-// LDS bytes a pass needs at least when its tail runs a small step (the
-// small step's region and the ticket flag); the launchers raise their
-// dynamic LDS to it.
-size_t pass_tail_lds(const PassArgs &a, size_t lds);
 
 constexpr int kPassRows = 32;
 constexpr int kPassMaxCols = 288;

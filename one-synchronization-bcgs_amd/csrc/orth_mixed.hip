@@ -270,7 +270,7 @@ hipError_t launch_pass16m_t(const PassArgs &a, size_t lds, int nwg, hipStream_t 
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    k_pass16m<NB, MX><<<dim3(nwg), dim3(kM), pass_tail_lds(a, lds), st>>>(a);
+    k_pass16m<NB, MX><<<dim3(nwg), dim3(kM), lds, st>>>(a);
     return hipGetLastError();
 }
 
@@ -387,7 +387,7 @@ hipError_t launch_pass16d_mixed_t(const PassArgs &a, int nwg, hipStream_t st)
         attr_set = true;
     }
     const size_t lds = (size_t)pass16d_lds(a.wl, NW) * sizeof(double);
-    k_pass16d<NW, NB, MX><<<dim3(nwg), dim3(64 * NW), pass_tail_lds(a, lds), st>>>(a);
+    k_pass16d<NW, NB, MX><<<dim3(nwg), dim3(64 * NW), lds, st>>>(a);
     return hipGetLastError();
 }
 

@@ -7,8 +7,7 @@
 // kept per device; host code uses only that address (the array's name is a
 // host-side stand-in, not a device address).  The address is carved into
 // the buffers of one call (factor slots, status, the synchronization
-// kernel's ticket counter, reduced projections, R, the small steps' work
-// matrix, the next pass's coefficients, and the projection partials, which
+// kernel's ticket counter, reduced projections, R, the next pass's coefficients, and the projection partials, which
 // take the rest).  Nothing is allocated: no hipMalloc, no event, no pinned
 // staging.  Every call on a device shares that device's array, and a call
 // clears what must start at zero with kernels (R, the factor slots, the
@@ -74,15 +73,12 @@ bool fixed_setup(FixedDev &f, int dev)
     Scratch &sc = f.sc;
     sc.stash = take(scratch_stash_need());
     sc.status_d = (int *)take(32);
-    sc.tickets_n = kTailTickets;
     sc.tickets = (int *)take(kTailTickets / 2);
     sc.P_n = scratch_p_need(kNoAllocMaxN);
     sc.P[0] = take(sc.P_n);
     sc.P[1] = take(sc.P_n);
     sc.Rd_n = scratch_r_need(kNoAllocMaxN);
     sc.Rd = take(sc.Rd_n);
-    sc.Tbig_n = scratch_tbig_need(kNoAllocMaxN);
-    sc.Tbig = take(sc.Tbig_n);
     sc.Cbuf_n = scratch_cbuf_need(kNoAllocMaxN);
     sc.Cbuf = take(sc.Cbuf_n);
     sc.part = q;

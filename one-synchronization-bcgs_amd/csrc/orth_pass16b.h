@@ -492,7 +492,7 @@ hipError_t launch_pass16b_v(const PassArgs &a, size_t lds, int nwg, hipStream_t 
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    k_pass16b<MT, NB, F, EARLY, V2, MX><<<dim3(nwg), dim3(kB), pass_tail_lds(a, lds), st>>>(a);
+    k_pass16b<MT, NB, F, EARLY, V2, MX><<<dim3(nwg), dim3(kB), lds, st>>>(a);
     return hipGetLastError();
 }
 

@@ -1,7 +1,6 @@
-// The synchronization at the end of a fused pass, inside the pass launch:
-// the fixed-order sum of the workgroups' projection partials and the small
-// step that follows it (the reference's MPI_Allreduce and the s x s work
-// after it, SRC/orth.c:114, :133, :188, :197).  Workgroups never wait for
+// The reduction at the end of a fused pass, inside the pass launch: the
+// fixed-order sum of the workgroups' projection partials (the reference's
+// MPI_Allreduce, SRC/orth.c:114, :133, :188, :197).  Workgroups never wait for
 // one another: each takes a ticket after storing its partial, and only the
 // last workgroup of a group (then the last group) goes on.
 #pragma once
@@ -10,12 +9,8 @@
 #include <stddef.h>
 
 #include "orth_kernels.h"
-#include "orth_small.h"
 
 namespace orth {
-
-// LDS of the tail: the small step's region and the ticket flag after it.
-constexpr size_t kTailLdsBytes = (size_t)(kSmallLds + 1) * sizeof(double);
 
 // Sum of the partials [k0, k1) of element e in workgroup order, starting
 // from the first (no added zero, so the sign of an exact zero is kept).
@@ -108,12 +103,12 @@ static __device__ __forceinline__ TailArgs tail_args(kernarg_ptr kp)
 }
 
 // Every thread of every workgroup of the pass calls this after its
-// workgroup's partial is stored; it returns at once unless the pass
-// synchronizes itself (PassArgs::tail_on).  stash: kernarg_stash() from the
+// workgroup's partial is stored; it returns at once unless the pass reduces
+// its own partials (PassArgs::tail_on).  stash: kernarg_stash() from the
 // kernel entry; nt: the workgroup's thread count (block size and grid size
 // come from the arguments, so that nothing of the dispatch stays live
-// through the pass).  sm: the pass's dynamic LDS, at least pass_tail_lds()
-// bytes; the pass no longer uses it.
+// through the pass).  sm: the pass's dynamic LDS (its first word is
+// the ticket flag); the pass no longer uses it.
 static __device__ __forceinline__ void pass_tail(const PassArgs &a, double *sm, uint64_t stash,
                                                  int nt)
 {
@@ -126,7 +121,7 @@ static __device__ __forceinline__ void pass_tail(const PassArgs &a, double *sm, 
     const int ngrp = (nwg + t.grp - 1) / t.grp;
     const int g = (int)blockIdx.x / t.grp;
     const int k0 = g * t.grp, k1 = min(nwg, k0 + t.grp);
-    int *flag = (int *)(sm + kSmallLds);
+    int *flag = (int *)sm;
 
     // The pass's own LDS and memory traffic is finished: tail_ticket waits
     // for every wave's loads and stores and synchronizes the workgroup.
@@ -141,9 +136,6 @@ static __device__ __forceinline__ void pass_tail(const PassArgs &a, double *sm, 
         for (int64_t e = threadIdx.x; e < E; e += nt)
             t.out[e] = part_range_sum(t.lvl, E, e, 0, ngrp);
     }
-    if (!t.small) return;
-    __syncthreads();
-    small_step(nt, t.sm, sm);
 }
 
 }  // namespace orth
