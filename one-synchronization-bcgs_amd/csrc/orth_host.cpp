@@ -137,12 +137,10 @@ bool ctx_init(DevCtx &c)
 // read at each call): part of the key of captured batch graphs.
 int64_t env_bits()
 {
-    static const char *const names[] = {"ORTH_UNFUSED", "ORTH_UPDATE_ROWWISE", "ORTH_PASS256",
-                                        "ORTH_GENERIC_PASS", "ORTH_MIXED_PASS32",
-                                        "ORTH_PASS_TILE32", "ORTH_PASS_LOAD8",
-                                        "ORTH_SEPARATE_REDUCE", "ORTH_PASS_REGPF", "ORTH_PASS16D_ONEWG",
-                                        "ORTH_PASS16D_MINCOLS", "ORTH_REDUCE_LAUNCH",
-                                        "ORTH_IN_PASS_SYNC"};
+    static const char *const names[] = {"ORTH_UNFUSED", "ORTH_UPDATE_ROWWISE", "ORTH_MIXED_PASS32",
+                                        "ORTH_SEPARATE_REDUCE", "ORTH_PASS_REGPF",
+                                        "ORTH_PASS16D_ONEWG", "ORTH_PASS16D_MINCOLS",
+                                        "ORTH_REDUCE_LAUNCH", "ORTH_IN_PASS_SYNC"};
     int64_t b = 0;
     for (int i = 0; i < (int)(sizeof(names) / sizeof(names[0])); i++)
         if (getenv(names[i])) b |= (int64_t)1 << i;
@@ -581,8 +579,6 @@ class Run {
     // Fraction of the device's workgroups one pass uses (the batched form
     // runs several calls side by side).
     void set_wg_scale(double f) { wg_scale_ = std::min(1.0, std::max(f, 1e-3)); }
-    // Column bound of the double-buffered s = 16 pass (0: the default).
-    void set_pass16d_min_cols(int c) { minc_ = std::max(0, c); }
     // Allow ORTH_IN_PASS_SYNC (the reduction inside the passes).
     void set_in_pass_sync(bool on) { in_pass_sync_ = on; }
 
@@ -627,9 +623,6 @@ class Run {
         pa.na = (int)na;
         pa.b0 = (int)(b0 - cb);
         pa.nb = (int)nb;
-        // Kernel choice: the 512-thread s = 16 pass when it applies, else the
-        // 256-thread passes (whose s = 16 form needs the tile padded to
-        // ceil(Ma / 4) projection tiles per wave).
         if (mx_) {
             // Columns at or past the written frontier still live only in X32.
             pa.X32 = x32_ + cb * ldx32_;
@@ -639,17 +632,14 @@ class Run {
             pa.lpb = lp_from_ >= 0 ? (int)(lp_from_ - cb) : (1 << 30);
         }
         int mt = 0, nbt = 0;
-        const int td = (S_ == 16 && !getenv("ORTH_PASS256") && !getenv("ORTH_MIXED_PASS32"))
-                           ? pass16d_plan(pa, &mt, &nbt, lp_first_pass(), minc_)
+        const int td = mx_ && !getenv("ORTH_MIXED_PASS32")
+                           ? pass16d_plan(pa, &mt, &nbt, lp_first_pass())
                            : 0;
-        const int ts16 = td > 0 ? 32
-                         : (S_ == 16 && !mx_ && !getenv("ORTH_PASS256")) ? pass16b_plan(pa, &mt, &nbt)
-                                                                          : 0;
         int64_t unit = kPassRows;
         int tsm = 0;
-        if (td > 0) {
-            unit = 32;
-        } else if (mx_) {
+        if (!mx_) {
+            unit = pass_rows(S_, pa);
+        } else if (td == 0) {
             // The 512-thread pass with super-tiles when the slab allows it,
             // else the 32-row mixed pass.
             tsm = getenv("ORTH_MIXED_PASS32") ? 0 : pass16bm_plan(pa);
@@ -657,22 +647,11 @@ class Run {
                 unit = tsm;
             else if (pass16m_lds_bytes(pa) == 0)
                 return nullptr;
-        } else if (ts16 > 0) {
-            unit = ts16;
-        } else if (S_ == 16 && na > 0) {
-            const int64_t mtp = ((na + 15) / 16 + 3) / 4;
-            pa.wl = (int)std::max<int64_t>(pa.wl, a0 - cb + 64 * mtp);
         }
-        if (!mx_ && td == 0 && ts16 == 0) unit = pass_rows(S_, pa);
-        // Two 512-thread workgroups per CU when the s = 16 pass applies (its
-        // LDS is under half a CU's), so one hides the other's barriers.
-        // The mixed pass with reduced-precision products runs one 512-thread
-        // workgroup per CU (its operand conversions need two waves' worth of
-        // registers); with FP64 products it runs two, like the FP64 pass.
-        // The 256-thread passes keep as many workgroups per CU as their
-        // registers and LDS allow.
-        // The double-buffered pass with 16 waves holds a whole CU (one
-        // workgroup).
+        // Workgroups per CU: the mixed pass with reduced-precision products
+        // runs one (its operand conversions need two waves' worth of
+        // registers), with FP64 products two, except the double-buffered one
+        // with 16 waves, which holds a whole CU.
         // One k_reduce_small launch after the pass sums its partials and runs
         // the small step.  ORTH_IN_PASS_SYNC=1 sums them in the pass's last
         // workgroups instead and launches only the small step after it, which
@@ -684,10 +663,9 @@ class Run {
         // The in-pass group sums follow the partials in `part`.
         bool tail = na > 0 && sc_.tickets && in_pass_sync_ && getenv("ORTH_IN_PASS_SYNC") &&
                     !getenv("ORTH_SEPARATE_REDUCE") && !getenv("ORTH_REDUCE_LAUNCH");
-        const int per_cu = td == 16                          ? 1
-                           : (ts16 > 0 || mx_ == kMxFP64) ? 2
-                           : mx_                           ? 1
-                                                           : pass_wg_per_cu(S_, pa, tail);
+        const int per_cu = !mx_                          ? pass_wg_per_cu(S_, pa, tail)
+                           : td != 16 && mx_ == kMxFP64 ? 2
+                                                        : 1;
         int nwg = std::max(1, (int)(std::max(1, c_.ncu) * per_cu * wg_scale_));
         if (na > 0 && sc_.fixed) {
             // Fixed scratch: fewer row chunks, so that the partials fit.
@@ -723,12 +701,10 @@ class Run {
             wcols += pend_.g[g].w;
         }
         if (!timed(c_, ORTH_K_PASS, st_, flops, 8.0 * m_ * (ncols + wcols), [&] {
-                if (td > 0) return mx_ ? launch_pass16d_mixed(pa, mx_, td, nbt, nwg, st_)
-                                       : launch_pass16d(pa, td, nbt, nwg, st_);
-                if (mx_)
-                    return tsm > 0 ? launch_pass16bm(pa, mx_, nwg, st_)
-                                   : launch_pass16m(pa, mx_, nwg, st_);
-                return ts16 > 0 ? launch_pass16b(pa, nwg, st_) : launch_pass(S_, pa, nwg, st_);
+                if (!mx_) return launch_pass(S_, pa, nwg, st_);
+                if (td > 0) return launch_pass16d_mixed(pa, mx_, td, nbt, nwg, st_);
+                return tsm > 0 ? launch_pass16bm(pa, mx_, nwg, st_)
+                               : launch_pass16m(pa, mx_, nwg, st_);
             }))
             return nullptr;
         for (int g = 0; g < pend_.ngrp; g++)
@@ -996,7 +972,6 @@ class Run {
     int64_t frontier_ = 0;      // columns [0, frontier_) have been written to X
     int64_t lp_from_ = -1;      // next pass: B columns from here on are reduced precision
     double wg_scale_ = 1.0;
-    int minc_ = 0;
     bool in_pass_sync_ = true;
 
     // Debug aid (ORTH_DEBUG_DUMP set): print the reduced projection and the
@@ -1146,7 +1121,7 @@ struct BatchCfg {
     int streams = 4;
     double wg_scale = 0.5;
     bool graph = true;  // capture into hipGraphs (else launch directly on the streams)
-    int minc = 0;       // column bound of the double-buffered s = 16 pass (0: default)
+    int minc = 0;       // field of the tuning cache's lines, without effect
 };
 
 // Graph nodes per captured graph at most: batches beyond it are captured as
@@ -1235,7 +1210,6 @@ std::vector<int64_t> full_key(const BatchArgs &a, const BatchCfg &cfg)
     k.push_back(cfg.graph ? 1 : 0);
     k.push_back(cfg.streams);
     k.push_back((int64_t)(cfg.wg_scale * 1e6));
-    k.push_back(cfg.minc);
     // Captured graphs hold the small steps' arguments, the shift among them,
     // and the kernels the environment switches selected.
     const double ps = g_pshift.load();
@@ -1350,7 +1324,6 @@ bool batch_enqueue(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg,
         for (int i : lists[k]) {
             Run r(b.slot[k], b.slot[k].sc, a.m[i], a.n[i], a.s[i], a.X[i], a.ldX[i], st);
             r.set_wg_scale(cfg.wg_scale);
-            r.set_pass16d_min_cols(cfg.minc);
             // Concurrent instances always reduce in a launch after each
             // pass: inside the passes, the last workgroups' acquires reach
             // into the L2 the other streams' instances are using.
@@ -1673,23 +1646,6 @@ bool batch_tune(BatchCtx &b, const BatchArgs &a, const InputBackup &bk, BatchCfg
                 best = ms;
                 bestc = cand;
             }
-        }
-    }
-    // Tile shape of the s = 16 passes, with the best placement: the
-    // double-buffered 32-row pass on every slab of 16 columns or more, or
-    // never (the 512-thread super-tile pass throughout), against the
-    // library's column bound.
-    for (const int mc : {16, 1 << 20}) {
-        if (!good) break;
-        BatchCfg cand = bestc;
-        cand.minc = mc;
-        good = bk.restore(a, b.main) && batch_run(b, a, cand) && bk.restore(a, b.main) &&
-               ok(hipEventRecord(e0, b.main)) && batch_run(b, a, cand) &&
-               ok(hipEventRecord(e1, b.main)) && ok(hipEventSynchronize(e1));
-        float ms = 0.f;
-        if (good && ok(hipEventElapsedTime(&ms, e0, e1)) && ms < best) {
-            best = ms;
-            bestc = cand;
         }
     }
     (void)hipEventDestroy(e0);

@@ -191,6 +191,7 @@ struct PassArgs {
     int seq;  // 1: group 1's product uses group 0's finished columns
     PassGroup g[2];
     int a0, na, b0, nb;  // step 2 ranges (na == 0: no projection)
+    int bsh;             // tile pass: columns its first N-tile starts before b0 (set by its launch)
     double *part;
     int64_t rows_per;
     // Mixed form only: columns >= raw0 (never written yet) are read from the
@@ -215,25 +216,22 @@ int pass_wg_per_cu(int S, const PassArgs &a, bool tail);
 // Rows per tile (the row-chunk unit) of the 256-thread passes for a.
 int pass_rows(int S, const PassArgs &a);
 
-// Block width 16 with 512 threads per workgroup: super-tile rows for the
-// pass (multiple of 32, 0 when it does not apply); rows_per must be a
-// multiple of it.
-int pass16b_plan(const PassArgs &a, int *mt, int *nb);
-size_t pass16b_lds_bytes(const PassArgs &a, int ts);
-hipError_t launch_pass16b(const PassArgs &a, int nwg, hipStream_t st);
+// The tile pass (orth_tpass.h), which launch_pass prefers: rows per tile or 0
+// when it does not apply, and its workgroups per CU.
+int tpass_rows(int S, const PassArgs &a);
+int tpass_wg_per_cu(int S, const PassArgs &a);
+hipError_t launch_tpass(int S, const PassArgs &a, int nwg, hipStream_t st);
 
-// Block width 16, FP64, double-buffered direct-to-LDS loads in 32-row tiles
+// Mixed form with double-buffered direct-to-LDS loads in 32-row tiles
 // (rows_per must be a multiple of 32): waves per workgroup (8 or 16), or 0
 // when it does not apply.
-// any_width: also below the column bound (the mixed form with reduced
-// precisions, whose 512-thread pass runs one workgroup per CU).  min_cols:
-// the column bound (0: the library's default; the batched form's tuner
-// picks it per batch).
+// any_width: also below the column bound (reduced precisions, whose
+// 512-thread pass runs one workgroup per CU).  min_cols: the column bound
+// (0: the library's default).
 int pass16d_plan(const PassArgs &a, int *mt, int *nb, bool any_width = false, int min_cols = 0);
-// Launch with the plan's waves per workgroup (nw) and N-tiles (nb).
-hipError_t launch_pass16d(const PassArgs &a, int nw, int nb, int nwg, hipStream_t st);
-// Its mixed form (a.X32 set): mx = kMxFP64 (FP32 storage, FP64 products) or
-// a reduced precision for the projection tiles from lpb on.
+// Launch with the plan's waves per workgroup (nw) and N-tiles (nb): mx =
+// kMxFP64 (FP32 storage, FP64 products) or a reduced precision for the
+// projection tiles from lpb on.
 hipError_t launch_pass16d_mixed(const PassArgs &a, int mx, int nw, int nb, int nwg,
                                 hipStream_t st);
 

@@ -1,5 +1,5 @@
-// The 256-thread fused passes (gfx950): the generic pass for any block width
-// and the s = 16 form with compile-time tile counts.
+// The fused pass for block widths 17 to 32 (256 threads), and the dispatch of
+// the FP64 passes: every narrower block runs the tile pass (orth_tpass.h).
 #include "orth_kernels.h"
 
 #include <stdlib.h>
@@ -38,21 +38,14 @@ size_t pass_lds_bytes(const PassArgs &a, int F)
     return ((size_t)a.wl * (F * kPT + 1) + (size_t)k1p * a.n1 + 2 * kMaxS * kMaxS) * sizeof(double);
 }
 
-// Waves per SIMD (= 256-thread workgroups per CU) the generic pass is
-// compiled for: the wide instance uses up to 512 registers per lane (one
-// workgroup per CU); the narrow one fits three (S <= 8) or two (S = 16).
-constexpr int pass_waves(int S, int MT) { return MT > 4 || S > 16 ? 1 : S <= 8 ? 3 : 2; }
-
-// MT: projection tiles per wave, PF: prefetch registers per thread.  The
-// narrow instance (fewer of both) fits several workgroups per CU.  V2: every
-// lane moves two consecutive rows with one 16-byte load (even ldX and m,
-// 16-byte aligned slab).  F: rows per tile = 32 F (the narrow instance with
-// few columns takes longer runs of each column per tile).
-template <int S, int MT = kPassMaxTiles, int PF = kPF, bool V2 = false, int F = 1>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-    pass_waves(S, MT), pass_waves(S, MT)))) void k_pass(PassArgs a)
+// One workgroup per CU (up to 512 registers per lane).  MT: projection tiles
+// per wave, PF: prefetch registers per thread.  V2: every lane moves two
+// consecutive rows with one 16-byte load (even ldX and m, 16-byte aligned
+// slab).
+template <int MT, int PF, bool V2>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_pass(PassArgs a)
 {
-    constexpr int TS = kPT * F, PLD = TS + 1;
+    constexpr int S = kMaxS, TS = kPT, PLD = TS + 1;
     extern __shared__ double sm[];
     const uint64_t kst = kernarg_stash();
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -259,341 +252,58 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     pass_tail(a, sm, kst, 256);
 }
 
-// Block width 16, the benchmark shape: compile-time tile counts, 32-bit
-// LDS offsets, four independent MFMA chains in step 1.  Wave w computes
-// Z tile (rows 16 (w & 1), cols 16 (w >> 1)) in step 1 and projection tiles
-// [w MT, (w+1) MT) x [0, NB) in step 2.
-template <int MT, int NB>
-__global__ __launch_bounds__(256) void k_pass16(PassArgs a)
-{
-    constexpr int S = 16, N1 = 32, LD = kPLd;
-    extern __shared__ double sm[];
-    const uint64_t kst = kernarg_stash();
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 15, lk = lane >> 4;
-    const int k1p = (a.k1 + 3) & ~3;
-    const int C0 = a.wl * LD, T0 = C0 + k1p * N1;
-
-    for (int e = tid; e < k1p * N1; e += 256) sm[C0 + e] = a.C[e];
-    for (int g = 0; g < a.ngrp; g++) {
-        const double *T = a.g[g].T;
-        const int w = a.g[g].w;
-        if (T)
-            for (int e = tid; e < S * S; e += 256) {
-                const int i = e % S, j = e / S;
-                sm[T0 + g * S * S + e] = (i < w && j < w) ? T[i + j * kLdT] : 0.0;
-            }
-    }
-    for (int e = tid; e < (a.wl - a.ncols) * kPT; e += 256)
-        sm[(a.ncols + e / kPT) * LD + (e % kPT)] = 0.0;
-
-    const int Ma = (a.na + 15) >> 4;
-    const bool proj = a.na > 0;
-    const int mt1 = wave & 1, nt1 = wave >> 1;
-    const int aoff1 = lk * LD + mt1 * 16 + li;
-    const int boff1 = C0 + lk * N1 + nt1 * 16 + li;
-    int aoff2[MT], boff2[NB];
-#pragma unroll
-    for (int i = 0; i < MT; i++) aoff2[i] = (a.a0 + (wave * MT + i) * 16 + li) * LD + lk;
-#pragma unroll
-    for (int j = 0; j < NB; j++) boff2[j] = (a.b0 + j * 16 + li) * LD + lk;
-
-    dbl4 acc[MT][NB];
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < NB; j++) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-
-    const int64_t rb = (int64_t)blockIdx.x * a.rows_per;
-    const int64_t re = min(a.m, rb + a.rows_per);
-    const int nload = a.ncols * kPT;
-    const double *Xl = a.X + (tid & (kPT - 1));
-    double pf[kPF];
-    auto load = [&](int64_t r0) {
-        const bool full = r0 + kPT <= re;
-#pragma unroll
-        for (int i = 0; i < kPF; i++) {
-            const int e = tid + 256 * i;
-            if (e < nload) {
-                const int64_t off = r0 + (int64_t)(e >> 5) * a.ldX;
-                pf[i] = (full || r0 + (e & 31) < re) ? Xl[off] : 0.0;
-            }
-        }
-    };
-    if (rb < re) load(rb);
-
-    for (int64_t r0 = rb; r0 < re; r0 += kPT) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kPF; i++) {
-            const int e = tid + 256 * i;
-            if (e < nload) sm[(e >> 5) * LD + (e & 31)] = pf[i];
-        }
-        __syncthreads();
-        if (r0 + kPT < re) load(r0 + kPT);
-
-        if (a.ngrp > 0) {
-            const int nphase = a.seq ? a.ngrp : 1;
-            for (int p = 0; p < nphase; p++) {
-                const int glo = a.seq ? p : 0, ghi = a.seq ? p + 1 : a.ngrp;
-                const int kp = a.seq ? ((a.g[p].k + 3) & ~3) : k1p;
-                const bool mine = a.k1 > 0 && (!a.seq || nt1 == (a.g[p].zoff >> 4));
-                dbl4 z = dbl4{0.0, 0.0, 0.0, 0.0};
-                if (mine) {
-                    dbl4 z1 = z, z2 = z, z3 = z;
-                    const int nks = kp >> 2;
-                    int ks = 0;
-                    for (; ks + 4 <= nks; ks += 4) {
-                        const int ao = aoff1 + 4 * ks * LD, bo = boff1 + 4 * ks * N1;
-                        const double x0 = sm[ao], x1 = sm[ao + 4 * LD], x2 = sm[ao + 8 * LD],
-                                     x3 = sm[ao + 12 * LD];
-                        const double c0 = sm[bo], c1 = sm[bo + 4 * N1], c2 = sm[bo + 8 * N1],
-                                     c3 = sm[bo + 12 * N1];
-                        z = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, c0, z, 0, 0, 0);
-                        z1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, c1, z1, 0, 0, 0);
-                        z2 = __builtin_amdgcn_mfma_f64_16x16x4f64(x2, c2, z2, 0, 0, 0);
-                        z3 = __builtin_amdgcn_mfma_f64_16x16x4f64(x3, c3, z3, 0, 0, 0);
-                    }
-                    for (; ks < nks; ks++)
-                        z = __builtin_amdgcn_mfma_f64_16x16x4f64(sm[aoff1 + 4 * ks * LD],
-                                                                 sm[boff1 + 4 * ks * N1], z, 0,
-                                                                 0, 0);
-                    z = (z + z1) + (z2 + z3);
-                }
-                __syncthreads();
-                if (mine) {
-                    const int zc = nt1 * 16 + li;
-                    for (int g = glo; g < ghi; g++) {
-                        const int off = zc - a.g[g].zoff;
-                        if (off >= 0 && off < a.g[g].w) {
-                            const int o = (a.g[g].t0 + off) * LD + mt1 * 16 + lk;
-#pragma unroll
-                            for (int v = 0; v < 4; v++) sm[o + 4 * v] -= z[v];
-                        }
-                    }
-                }
-                __syncthreads();
-                // Row-wise forward substitution (dtrsm_('R','U','N','N')).
-                if (tid < (ghi - glo) * kPT) {
-                    const int g = glo + tid / kPT, row = tid % kPT;
-                    if (a.g[g].T) {
-                        const int w = a.g[g].w;
-                        const int o = a.g[g].t0 * LD + row;
-                        const int tg = T0 + g * S * S;
-                        double x[S];
-#pragma unroll
-                        for (int i = 0; i < S; i++) x[i] = i < w ? sm[o + i * LD] : 0.0;
-#pragma unroll
-                        for (int i = 0; i < S; i++) {
-                            if (i < w) {
-                                double v = x[i];
-#pragma unroll
-                                for (int l = 0; l < i; l++) v = fma(-x[l], sm[tg + l + i * S], v);
-                                x[i] = v * (1.0 / sm[tg + i + i * S]);
-                            }
-                        }
-#pragma unroll
-                        for (int i = 0; i < S; i++)
-                            if (i < w) sm[o + i * LD] = x[i];
-                    }
-                }
-                __syncthreads();
-            }
-            for (int g = 0; g < a.ngrp; g++) {
-                const int t0 = a.g[g].t0;
-                for (int e = tid; e < a.g[g].w * kPT; e += 256) {
-                    const int cc = e >> 5, rr = e & 31;
-                    if (r0 + rr < re)
-                        a.X[r0 + rr + (int64_t)(t0 + cc) * a.ldX] = sm[(t0 + cc) * LD + rr];
-                }
-            }
-        }
-
-        if (proj) {
-#pragma unroll
-            for (int ks = 0; ks < kPT / 4; ks++) {
-                double bv[NB], av[MT];
-#pragma unroll
-                for (int j = 0; j < NB; j++) bv[j] = sm[boff2[j] + 4 * ks];
-#pragma unroll
-                for (int i = 0; i < MT; i++) av[i] = sm[aoff2[i] + 4 * ks];
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NB; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i], bv[j], acc[i][j],
-                                                                        0, 0, 0);
-            }
-        }
-    }
-
-    if (proj) {
-        double *out = a.part + (int64_t)blockIdx.x * a.na * a.nb;
-#pragma unroll
-        for (int i = 0; i < MT; i++) {
-            const int ta = wave * MT + i;
-            if (ta < Ma) {
-#pragma unroll
-                for (int j = 0; j < NB; j++) {
-                    const int col = j * 16 + li;
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int row = ta * 16 + lk + 4 * v;
-                        if (row < a.na && col < a.nb) out[row + (int64_t)col * a.na] = acc[i][j][v];
-                    }
-                }
-            }
-        }
-    }
-    pass_tail(a, sm, kst, 256);
-}
-
-// Tiles per wave of the s = 16 kernel for a pass, or 0 when it does not apply.
-static int pass16_mt(const PassArgs &a)
-{
-    if (a.n1 != 32) return 0;
-    if (a.na == 0) return 1;
-    const int Ma = (a.na + 15) / 16, Nb = (a.nb + 15) / 16;
-    if (Nb > 2) return 0;
-    const int mt = (Ma + 3) / 4;
-    if (mt > 5 || a.a0 + 64 * mt > a.wl) return 0;
-    return mt;
-}
-
-template <int MT, int NB>
-hipError_t launch_pass16_t(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
-{
-    static bool attr_set = false;
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)k_pass16<MT, NB>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)(160 * 1024));
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
-    k_pass16<MT, NB><<<dim3(nwg), dim3(256), lds, st>>>(a);
-    return hipGetLastError();
-}
-
-hipError_t launch_pass16(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
-{
-    const int mt = pass16_mt(a);
-    const int nb = a.na > 0 ? (a.nb + 15) / 16 : 1;
-#define ORTH_P16(M)                                                                  \
-    case M:                                                                          \
-        return nb == 2 ? launch_pass16_t<M, 2>(a, lds, nwg, st)                     \
-                       : launch_pass16_t<M, 1>(a, lds, nwg, st);
-    switch (mt) {
-        ORTH_P16(1)
-        ORTH_P16(2)
-        ORTH_P16(3)
-        ORTH_P16(4)
-        ORTH_P16(5)
-    default: return hipErrorInvalidValue;
-    }
-#undef ORTH_P16
-}
-
-// The narrow generic pass: at most kNarrowCols columns and 4 projection
-// tiles per wave.
+// The narrow instance: at most kNarrowCols columns and 4 projection tiles
+// per wave.
 constexpr int kNarrowCols = 160;
 constexpr int kNarrowPF = kNarrowCols * kPT / 256;
 
-bool pass_narrow(const PassArgs &a)
+static bool pass_narrow(const PassArgs &a)
 {
     const int Ma = (a.na + 15) / 16, Nb = (a.nb + 15) / 16;
     return a.ncols <= kNarrowCols && (a.na == 0 || Ma * Nb <= 4 * 4);
 }
 
-template <int S, int MT, int PF, bool V2 = false, int F = 1>
-hipError_t launch_pass_v(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
+// Two-row (16-byte) loads: even leading dimension and row count, 16-byte
+// aligned slab.
+static bool pass_v2_ok(const PassArgs &a)
+{
+    return a.ldX % 2 == 0 && a.m % 2 == 0 && (uintptr_t)a.X % 16 == 0;
+}
+
+template <int MT, int PF, bool V2>
+static hipError_t launch_pass_v(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
 {
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)k_pass<S, MT, PF, V2, F>,
+        hipError_t e = hipFuncSetAttribute((const void *)k_pass<MT, PF, V2>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(160 * 1024));
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    k_pass<S, MT, PF, V2, F><<<dim3(nwg), dim3(256), lds, st>>>(a);
+    k_pass<MT, PF, V2><<<dim3(nwg), dim3(256), lds, st>>>(a);
     return hipGetLastError();
-}
-
-// Rows per tile of the generic pass, 32 F: the narrow instance takes F = 4
-// (S <= 8) or 2 (S <= 16) when the tile's columns fit its prefetch
-// registers (ncols * 32 F <= 256 * kNarrowPF) and the step-1 tiles fit.
-int pass_f(int S, const PassArgs &a)
-{
-    if (!pass_narrow(a) || getenv("ORTH_PASS_TILE32")) return 1;
-    for (int F = S <= 8 ? 4 : S <= 16 ? 2 : 1; F > 1; F >>= 1)
-        if (a.ncols * kPT * F <= 256 * kNarrowPF && pass_lds_bytes(a, F) != 0) return F;
-    return 1;
 }
 
 int pass_rows(int S, const PassArgs &a)
 {
-    if (S == 16 && pass16_mt(a) > 0 && !getenv("ORTH_GENERIC_PASS")) return kPT;  // k_pass16
-    return kPT * pass_f(S, a);
-}
-
-// Two-row (16-byte) loads: even leading dimension and row count, 16-byte
-// aligned slab.
-bool pass_v2_ok(const PassArgs &a)
-{
-    return a.ldX % 2 == 0 && a.m % 2 == 0 && (uintptr_t)a.X % 16 == 0 &&
-           !getenv("ORTH_PASS_LOAD8");
-}
-
-template <int S, int F>
-hipError_t launch_pass_n(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
-{
-    return pass_v2_ok(a) ? launch_pass_v<S, 4, kNarrowPF, true, F>(a, lds, nwg, st)
-                         : launch_pass_v<S, 4, kNarrowPF, false, F>(a, lds, nwg, st);
-}
-
-template <int S>
-hipError_t launch_pass_t(const PassArgs &a, int nwg, hipStream_t st)
-{
-    const int F = pass_f(S, a);
-    const size_t lds = pass_lds_bytes(a, F);
-    if (lds == 0 || a.rows_per % (kPT * F) != 0) return hipErrorInvalidValue;
-    if (pass_narrow(a)) {
-        if constexpr (S <= 8)
-            if (F == 4) return launch_pass_n<S, 4>(a, lds, nwg, st);
-        if constexpr (S <= 16)
-            if (F == 2) return launch_pass_n<S, 2>(a, lds, nwg, st);
-        return launch_pass_n<S, 1>(a, lds, nwg, st);
-    }
-    return launch_pass_v<S, kPassMaxTiles, kPF>(a, lds, nwg, st);
+    const int ts = tpass_rows(S, a);
+    return ts > 0 ? ts : kPT;
 }
 
 int pass_wg_per_cu(int S, const PassArgs &a, bool)
 {
-    const size_t lds = pass_lds_bytes(a, pass_f(S, a));
-    if (lds == 0) return 1;
-    // Register-limited residency (k_pass16 and the wide generic pass: one
-    // workgroup per CU).
-    const bool p16 = S == 16 && pass16_mt(a) > 0 && !getenv("ORTH_GENERIC_PASS");
-    const int by_regs = p16 ? 1 : pass_narrow(a) ? pass_waves(S, 4) : pass_waves(S, kPassMaxTiles);
-    const int by_lds = (int)std::max<size_t>(1, (160 * 1024) / lds);
-    return std::max(1, std::min(by_regs, by_lds));
+    return tpass_rows(S, a) > 0 ? tpass_wg_per_cu(S, a) : 1;
 }
 
 hipError_t launch_pass(int S, const PassArgs &a, int nwg, hipStream_t st)
 {
-    if (S == 16 && pass16_mt(a) > 0 && !getenv("ORTH_GENERIC_PASS")) {
-        const size_t lds = pass_lds_bytes(a);
-        if (lds == 0) return hipErrorInvalidValue;
-        return launch_pass16(a, lds, nwg, st);
-    }
-    switch (S) {
-    case 4: return launch_pass_t<4>(a, nwg, st);
-    case 8: return launch_pass_t<8>(a, nwg, st);
-    case 16: return launch_pass_t<16>(a, nwg, st);
-    case 32: return launch_pass_t<32>(a, nwg, st);
-    default: return hipErrorInvalidValue;
-    }
+    if (tpass_rows(S, a) > 0) return launch_tpass(S, a, nwg, st);
+    const size_t lds = pass_lds_bytes(a);
+    if (S != kMaxS || lds == 0 || a.rows_per % kPT != 0) return hipErrorInvalidValue;
+    if (!pass_narrow(a)) return launch_pass_v<kPassMaxTiles, kPF, false>(a, lds, nwg, st);
+    return pass_v2_ok(a) ? launch_pass_v<4, kNarrowPF, true>(a, lds, nwg, st)
+                         : launch_pass_v<4, kNarrowPF, false>(a, lds, nwg, st);
 }
 
 }  // namespace orth
