@@ -663,7 +663,7 @@ class Run {
         // The in-pass group sums follow the partials in `part`.
         bool tail = na > 0 && sc_.tickets && in_pass_sync_ && getenv("ORTH_IN_PASS_SYNC") &&
                     !getenv("ORTH_SEPARATE_REDUCE") && !getenv("ORTH_REDUCE_LAUNCH");
-        const int per_cu = !mx_                          ? pass_wg_per_cu(S_, pa, tail)
+        const int per_cu = !mx_                          ? pass_wg_per_cu(S_, pa)
                            : td != 16 && mx_ == kMxFP64 ? 2
                                                         : 1;
         int nwg = std::max(1, (int)(std::max(1, c_.ncu) * per_cu * wg_scale_));
@@ -766,21 +766,10 @@ class Run {
     // largest coefficient block: (n + s) x n1.
     bool fused_fits() const
     {
-        // The generic fused pass addresses up to four columns with 32-bit
-        // lane offsets.
-        if (ldX_ >= ((int64_t)1 << 27)) return false;
-        PassArgs pa;
-        memset(&pa, 0, sizeof(pa));
-        pa.ncols = (int)n_;
-        pa.wl = (int)((n_ + 15) / 16 * 16);
-        pa.k1 = (int)std::min<int64_t>(n_, pa.wl);
-        pa.n1 = n1_;
-        const int64_t Mt = (n_ + 15) / 16;
-        pa.na = (int)std::min<int64_t>(n_, Mt * 16);
-        pa.nb = (int)std::min<int64_t>(n_, 2 * s_);
-        pa.a0 = 0;
-        pa.b0 = (int)(pa.wl - ((pa.nb + 15) / 16) * 16);
-        return pass_lds_bytes(pa) != 0;
+        // The mixed passes address up to four columns with 32-bit lane offsets;
+        // the tile pass has the same bound.
+        if (S_ != kMaxS && ldX_ >= ((int64_t)1 << 27)) return false;
+        return pass_fits(S_, n_);
     }
 
     bool intra_qr_f(int64_t blk, int64_t col0, int64_t w, double *Rdst, int64_t ldRdst,

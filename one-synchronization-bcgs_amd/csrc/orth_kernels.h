@@ -204,23 +204,32 @@ struct PassArgs {
     TailArgs tail;
 };
 
-constexpr int kPassRows = 32;
-constexpr int kPassMaxCols = 288;
-
-// LDS bytes the fused pass needs, or 0 when the shape does not fit it.
-size_t pass_lds_bytes(const PassArgs &a, int F = 1);
-hipError_t launch_pass(int S, const PassArgs &a, int nwg, hipStream_t st);
-// Workgroups per CU the generic pass for this shape can keep resident (tail:
-// the pass runs its synchronization, whose LDS it then holds).
-int pass_wg_per_cu(int S, const PassArgs &a, bool tail);
-// Rows per tile (the row-chunk unit) of the 256-thread passes for a.
+// The FP64 passes (orth_pass.hip): does a call with n columns of block width
+// S fit them; rows per tile (the unit of a row chunk) and workgroups per CU
+// for a; launch.
+constexpr int kPassRows = 32;  // rows per tile of the mixed form
+bool pass_fits(int S, int64_t n);
 int pass_rows(int S, const PassArgs &a);
+int pass_wg_per_cu(int S, const PassArgs &a);
+hipError_t launch_pass(int S, const PassArgs &a, int nwg, hipStream_t st);
 
-// The tile pass (orth_tpass.h), which launch_pass prefers: rows per tile or 0
-// when it does not apply, and its workgroups per CU.
+// The tile pass (orth_tpass.h) for S <= 16 and the wide-block pass
+// (orth_wpass.h) for S = 32: rows are 0 for arguments they do not take.
+constexpr int kTpassMaxCols = 288;
 int tpass_rows(int S, const PassArgs &a);
 int tpass_wg_per_cu(int S, const PassArgs &a);
 hipError_t launch_tpass(int S, const PassArgs &a, int nwg, hipStream_t st);
+constexpr int kWpassMaxCols = 512;
+// Its coefficients: entry (k, n) of C (64 columns), in the order its lanes
+// hold them (one 16 x 16 tile: lane 16 (k % 4) + n % 16 holds rows k % 4 + 4 v).
+constexpr int kWpassN1 = 64;
+static inline __host__ __device__ int wpass_cidx(int k, int n)
+{
+    return (k >> 4) * (16 * kWpassN1) + (n >> 4) * 256 + ((k & 3) * 16 + (n & 15)) * 4 + ((k >> 2) & 3);
+}
+int wpass_rows(int S, const PassArgs &a);
+int wpass_wg_per_cu(int S, const PassArgs &a);
+hipError_t launch_wpass(int S, const PassArgs &a, int nwg, hipStream_t st);
 
 // Mixed form with double-buffered direct-to-LDS loads in 32-row tiles
 // (rows_per must be a multiple of 32): waves per workgroup (8 or 16), or 0

@@ -37,7 +37,6 @@
 
 namespace orth {
 
-constexpr int kTpMaxCols = 288;   // columns of a tile (16-row tiles)
 constexpr int kTpBuf = 4096;      // doubles per tile buffer with more than 16 rows
 
 // Step-1 split for TS rows and ZN 16-column tiles of Z.  The inner dimension
@@ -48,7 +47,7 @@ struct TpZ {
     static constexpr int ZI = ZT > NW ? ZT / NW : 1;        // tiles per wave
     static constexpr int KS = ZT < NW ? NW / ZT : 1;        // inner-dimension split
     static constexpr int MaxU =
-        (WIDE ? kTpMaxCols : NW == 16 || TS == 16 ? 256 : kTpBuf / TS) / 16;
+        (WIDE ? kTpassMaxCols : NW == 16 || TS == 16 ? 256 : kTpBuf / TS) / 16;
     static constexpr int UQ = (MaxU + KS - 1) / KS;  // units per wave
     static constexpr int Zs = (KS - 1) * ZT * 256;   // doubles of partial Z tiles
 };

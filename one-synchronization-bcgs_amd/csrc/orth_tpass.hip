@@ -16,7 +16,7 @@ struct TpPlan {
     int bsh = 0;  // columns the first N-tile of the projection starts before b0
 };
 
-// Block widths up to 16, FP64 columns, at most kTpMaxCols of them.
+// Block widths up to 16, FP64 columns, at most kTpassMaxCols of them.
 //
 // Rows per tile: two workgroups share a CU, so a buffer of TS rows takes
 // TS wl <= kTpBuf doubles (16-row tiles: up to 256 columns); fewer where the
@@ -43,7 +43,7 @@ TpPlan plan(int S, const PassArgs &a)
         p.bsh = std::max(0, a.b0 + 16 * Nb - wl);
     }
     wl = (wl + 15) / 16 * 16;
-    if (wl > kTpMaxCols) return p;
+    if (wl > kTpassMaxCols) return p;
     for (int g = 0; g < a.ngrp; g++)
         if (a.g[g].t0 + a.g[g].w > a.ncols || a.g[g].zoff % 4 != 0 ||
             a.g[g].zoff / 16 != (a.g[g].zoff + a.g[g].w - 1) / 16)
