@@ -339,7 +339,7 @@ static __device__ __forceinline__ void d_r_rows(int nt, int wlo, int mode, int c
 }
 
 // Every wave: coefficients of the next fused pass, row-major C[k][n] (ld n1;
-// n1 = 64: in the order of wpass_cidx) for k < roundup4(k1), in 16 x 16 tiles: columns [0, w0) are Y over rows
+// W = 32: in the order of wpass_cidx) for k < roundup4(k1), in 16 x 16 tiles: columns [0, w0) are Y over rows
 // [0, c), zero below; columns [S, S + w1) are S_top over rows [0, c) (with
 // sub: S_top - Y Z) and the w0 x w1 block Z in LDS (ld lz) over rows
 // [c, c + w0); everything else is zero.
@@ -373,7 +373,7 @@ static __device__ __forceinline__ void d_emit(int nt, double *C, int n1, int S, 
                 double x = 0.0;
                 if (jok && k < c) x = P[k + (int64_t)col * na] - z[v];
                 if (jok && g1 && k >= c && k < c + w0) x = Z[(k - c) * lz + j];
-                C[n1 == kWpassN1 ? wpass_cidx(k, n) : k * n1 + n] = x;
+                C[W == 32 ? wpass_cidx(k, n) : k * n1 + n] = x;
             }
         }
     }

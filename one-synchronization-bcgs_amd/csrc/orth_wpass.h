@@ -119,8 +119,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
         for (int v = 0; v < 4; v++) asm volatile("" ::"v"(cf[u][v]));
 
-    // Projection: M-tiles m0 + NW i, all NB N-tiles.
-    const int Ma = (a.na + 15) >> 4, m0 = NW - 1 - wave;
+    // Projection: M-tiles m0 + NW i, all NB N-tiles; the waves on the solving
+    // waves' SIMDs (the even ones), then those themselves, get the last ones.
+    const int Ma = (a.na + 15) >> 4;
+    const int m0 = wave & 1 ? wave >> 1 : NW / 2 + (NW == 8 ? (wave >> 1) ^ 2 : wave >> 1);
     const bool proj = a.na > 0 && m0 < Ma;
     // The N-tiles end with the buffer where they would leave it.
     const int b0 = a.b0 - a.bsh;
@@ -131,8 +133,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
         for (int t = 0; t < NB; t++) acc[i][t] = dbl4{0.0, 0.0, 0.0, 0.0};
     const bool hasg = a.ngrp > 0;
+    // The next tile's loads are issued at the tile's start when no solve or
+    // no projection follows; otherwise after step 1 (whose L2 reads would wait
+    // behind them), kEB before each M-tile during the solve and kFB before each
+    // after it: a CU takes about 9 bytes per cycle, and a wave that finds the
+    // path full stands still.  2^22 x 512, kEB / kFB: 1/1 116.2 ms, 1/2 118.1,
+    // 2/1 123.5, 3/0 121.1, 0/1 and the rest at the end 129.0.
+    const bool late = hasg && a.na > 0;
+    constexpr int kEB = 1, kFB = 1;
     // M-tiles (bit i) whose product with the N-tiles from 2 on touches no
-    // group's columns: taken before the solve is waited for.
+    // group's columns: the waves that do not solve take it during the solve.
     auto clean = [&](int c0, int c1) {
         bool r = true;
         for (int g = 0; g < a.ngrp; g++) {
@@ -142,7 +152,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         return r;
     };
     int early = 0;
-    if (NB == 4 && hasg && proj && clean(b0 + 32, b0 + 64)) {
+    if (NB == 4 && hasg && proj && !solver && clean(b0 + 32, b0 + 64)) {
 #pragma unroll
         for (int i = 0; i < MT; i++) {
             const int c0 = a.a0 + 16 * (m0 + NW * i);
@@ -157,23 +167,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int nfull = re > rb ? (int)((re - rb) / TS) : 0;
 
     // Loads (as in the tile pass): span i covers 64 consecutive 16-byte slots,
-    // CS columns; the spans go round the waves that do not solve.
+    // CS columns; the spans go round the waves.
     constexpr int CS = 128 / TS;
     const bool st16 = a.ldX % 2 == 0 && (uintptr_t)a.X % 16 == 0;
     const int nspan = (a.ncols + CS - 1) / CS;
-    int iw = wave, niw = NW;  // rank and number of the issuing waves
-    for (int w = 0; w < NW && hasg; w++) {
-        // Waves whose slice and half are the first and whose group exists solve.
-        const int wz = w % ZP::ZT % ZN;
-        if (w / ZP::ZT == 0 && (wz & 1) == 0 && wz / 2 < a.ngrp) {
-            niw--;
-            if (w < wave) iw--;
-        }
-    }
-    const int nsp = solver || iw >= nspan ? 0 : (nspan - iw + niw - 1) / niw;  // this wave's spans
-    const int ldc = CS * iw + lane / (TS / 2), ls = lane & (TS / 2 - 1);
+    const int nsp = nspan > wave ? (nspan - wave + NW - 1) / NW : 0;  // this wave's spans
+    const int ldc = CS * wave + lane / (TS / 2), ls = lane & (TS / 2 - 1);
     const char *gb = (const char *)(a.X + rb + (int64_t)ldc * a.ldX);
-    const int64_t gs = (int64_t)CS * niw * a.ldX * 8;
+    const int64_t gs = (int64_t)CS * NW * a.ldX * 8;
     const int ncols = a.ncols;
     // This wave's spans [j0, j1) of tile t into buf.
     auto issue = [&](int t, double *buf, int j0, int j1) {
@@ -181,8 +182,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         j1 = min(j1, nsp);
         if (st16) {
             const char *g = gb + (int64_t)t * (TS * 8) + j0 * gs;
-            int c = ldc + j0 * CS * niw, i = iw + j0 * niw;
-            for (int j = j0; j < j1; j++, g += gs, c += CS * niw, i += niw)
+            int c = ldc + j0 * CS * NW, i = wave + j0 * NW;
+            for (int j = j0; j < j1; j++, g += gs, c += CS * NW, i += NW)
                 if (c < ncols)
                     __builtin_amdgcn_global_load_lds((tp_glb_t *)(g + 16 * (ls ^ tswz<TS>(c))),
                                                      (tp_lds_t *)(buf + i * 128), 16, 0, 0);
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             const double *Xr = a.X + rb + (int64_t)t * TS;
             for (int j = j0; j < j1; j++)
                 for (int q = 0; q < 4; q++) {
-                    const int i = iw + j * niw;
+                    const int i = wave + j * NW;
                     const int e = 16 * q + (ln >> 2), s = e & (TS / 2 - 1);
                     const int c = i * CS + e / (TS / 2);
                     if (c < ncols)
@@ -203,13 +204,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
     };
     issue(0, sm, 0, nsp);
-
-    // The next tile's loads are issued at the tile's start when no solve or
-    // no projection follows; otherwise after step 1 (whose L2 reads would wait
-    // behind them), sb spans before each M-tile of the early products, which
-    // keep the matrix cores busy while the address path is.
-    const bool late = hasg && a.na > 0;
-    const int sb = (nsp + MT - 1) / MT;
 
     for (int t = 0; t < nt; t++) {
         double *cur = sm + (t & 1) * tsz;
@@ -275,6 +269,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     for (int i = 0; i < ZI; i++)
                         z[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[v], av[i][v], z[i], 0, 0, 0);
             };
+            // The upper half of the waves would finish last, alone on its SIMDs
+            // (the older wave goes first); this way round measured 0.5 % less.
+            if (NW == 8 && wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
             if (nun > 0) {
                 double av[ZI][4];
 #pragma unroll
@@ -330,6 +327,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         }
                 }
             }
+            if (NW == 8) __builtin_amdgcn_s_setprio(0);
             // Hand the Z tiles to the collecting waves: partials through LDS,
             // or (one slice) a group's second tile by subtracting it in place.
             if constexpr (KS > 1) {
@@ -456,7 +454,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
 #pragma unroll
             for (int i = 0; i < MT; i++) {
-                if (late && i * sb < nsp) issue(t + 1, nxt, i * sb, (i + 1) * sb);
+                if (late) issue(t + 1, nxt, kEB * i, kEB * (i + 1));
                 if (NB == 4 && (early >> i & 1)) project(acc[i], i, NB - 2);
             }
             tp_barrier();
@@ -483,9 +481,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
         }
 
-        if (proj) {
+        if (a.na > 0) {
 #pragma unroll
             for (int i = 0; i < MT; i++) {
+                if (late) issue(t + 1, nxt, kEB * MT + kFB * i, i + 1 < MT ? kEB * MT + kFB * (i + 1) : nsp);
                 if (m0 + NW * i < Ma) project(acc[i], i, 0);
                 if (NB == 4 && m0 + NW * i < Ma && !(early >> i & 1)) project(acc[i], i, NB - 2);
             }
