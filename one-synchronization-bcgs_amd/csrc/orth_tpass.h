@@ -128,12 +128,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const int ulo = nu * ksp / KS, nun = nu * (ksp + 1) / KS - ulo;
     const int uf = ulo + nun == nu ? nu - 1 : ulo;  // the first unit taken
     const int ur = uf == ulo ? ulo + 1 : ulo;       // start of the others
-    // This lane's Z column and the group column it belongs to (lv: any).
+    // This lane's Z column as an operand row, and its group (lv: any).
     const int zc = 16 * zn + li;
     const int gl = a.ngrp == 2 && zc >= a.g[1].zoff ? 1 : 0;
     const int goff = zc - ORTH_G(a, gl, zoff);
     const bool lv = gl < a.ngrp && goff >= 0 && goff < ORTH_G(a, gl, w);
-    const int lcol = lv ? ORTH_G(a, gl, t0) + goff : 0;
     const int cfin = SEQ ? a.g[0].t0 : 0;  // first finished column of the sequential form
     double cf[UQ][4];
 #pragma unroll
@@ -149,24 +148,25 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const int zf = tpos<TS>(16 * uf + lk, 16 * zm0 + li);
     const int zr = tpos<TS>(16 * ur + lk, 16 * zm0 + li);
     const int kc = 16 * uf + 16 > a.k1 ? a.k1 - 1 : 1 << 20;  // column clamp of unit uf
-    // Solve operands, held for the pass: B fragments (lane: row lk, column
-    // li) of the row blocks of the four 4-column blocks, each of one group;
+    // The Z tile is computed transposed (lane: row li of the chunk, columns
+    // lk + 4 v), so that value v of the chunk is the operand of block v of the
+    // blocked solve.  xi: the index of column lk + 4 v, or -1 past its group.
+    // Solve operands, held for the pass: A fragments (lane: column li, row
+    // lk) of the row blocks of the four 4-column blocks, each of one group;
     // zero in the other group's lanes.  smask: blocks to solve, group 0 in
     // bits 0-3, group 1 in bits 4-7.
     const bool solver = ksp == 0 && zany;
     double bw[4];
-    int ab[4], smask = 0;
+    int xi[4], smask = 0;
 #pragma unroll
     for (int b = 0; b < 4; b++) {
         const int zb = 16 * zn + 4 * b;
         const int gb = a.ngrp == 2 && zb >= a.g[1].zoff ? 1 : 0;
-        const int ob = zb - ORTH_G(a, gb, zoff), gw = ORTH_G(a, gb, w);
-        const double *T = gb < a.ngrp && ob < gw ? ORTH_G(a, gb, T) : nullptr;
+        const int ob = zb - ORTH_G(a, gb, zoff), gw = gb < a.ngrp ? ORTH_G(a, gb, w) : 0;
+        const double *T = ob < gw ? ORTH_G(a, gb, T) : nullptr;
         if (T) smask |= 1 << (b + 4 * gb);
         bw[b] = T && gl == gb && goff >= 0 ? T[kSlotW + 32 * ob + lk * kLdT + goff] : 0.0;
-        // A operand: row li of the block's column lk (columns past the group:
-        // its last column, with a zero row of B).
-        ab[b] = T ? tpos<TS>(ORTH_G(a, gb, t0) + min(ob + lk, gw - 1), 16 * zm0 + li) : 0;
+        xi[b] = ob + lk < gw ? tpos<TS>(ORTH_G(a, gb, t0) + ob + lk, 16 * zm0 + li) : -1;
     }
     // Sequential form: the second group's coefficients on the first group's
     // columns, row k at sfl + 16 k (lane: its Z column).
@@ -182,7 +182,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     }
     smask = __builtin_amdgcn_readfirstlane(smask);
     const int gsplit = a.ngrp == 2 ? a.g[1].zoff / 4 - 4 * zn : 4;  // first block of group 1
-    const int xb = tpos<TS>(lcol, 16 * zm0 + lk);  // the chunk's row lk + 4 v: XOR 4 v
     // Make the compiler wait for these loads here, once.
 #pragma unroll
     for (int u = 0; u < UQ; u++)
@@ -293,7 +292,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             dbl4 z[ZI];
 #pragma unroll
             for (int i = 0; i < ZI; i++) z[i] = dbl4{0.0, 0.0, 0.0, 0.0};
-            // A operand of a k-step: row 16 zm + li of its column lk.
+            // B operand of a k-step: row 16 zm + li of its column lk.
             auto unit = [&](int u, const double *const (&p)[4], int o) {
                 double av[ZI][4];
 #pragma unroll
@@ -305,7 +304,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 for (int v = 0; v < 4; v++)
 #pragma unroll
                     for (int i = 0; i < ZI; i++)
-                        z[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i][v], cf[u][v], z[i], 0, 0,
+                        z[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(cf[u][v], av[i][v], z[i], 0, 0,
                                                                    0);
             };
             if (nun > 0) {
@@ -335,28 +334,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             }
             tp_barrier();
             if (late) issue(t + 1, nxt);
-            // Chunk zm of the groups of tile zn in MFMA accumulator layout
-            // (lane: its column, rows 16 zm + lk + 4 v), minus the
-            // fixed-order sum of the partial Z tiles; then the blocked
-            // triangular solve, each block's columns through LDS once to
-            // become an A operand.
-            const int xq = tp_opaque(xb);
-            auto blocks = [&](dbl4 &x, int o, int mask) {
+            // Chunk zm of the groups of tile zn, minus the fixed-order sum of
+            // the partial Z tiles; then the blocked triangular solve, whose
+            // chain is its MFMAs alone.
+            auto blocks = [&](dbl4 &x, int mask) {
 #pragma unroll
                 for (int b = 0; b < 4; b++) {
                     if (!(mask >> b & 1)) continue;
-                    if ((liq >> 2) == b && lv) {
-#pragma unroll
-                        for (int v = 0; v < 4; v++) cur[(xq ^ (4 * v)) + o] = x[v];
-                    }
-                    tp_wave_fence();
-                    const double av = cur[ab[b] + o];
                     const dbl4 x0 = x;
-                    if ((liq >> 2) == b) x = dbl4{0.0, 0.0, 0.0, 0.0};
-                    x = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bw[b], x, 0, 0, 0);
+                    x[b] = 0.0;
+                    x = __builtin_amdgcn_mfma_f64_16x16x4f64(bw[b], x0[b], x, 0, 0, 0);
                     // Two groups in one tile: the other group's columns keep
                     // their values (0 times a NaN of this group is NaN).
-                    if (ZN == 1 && gl != (b >= gsplit ? 1 : 0)) x = x0;
+                    if (ZN == 1) {
+#pragma unroll
+                        for (int v = 0; v < 4; v++)
+                            if ((v >= gsplit) != (b >= gsplit)) x[v] = x0[v];
+                    }
                 }
             };
             dbl4 x[ZI];
@@ -365,7 +359,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 for (int i = 0; i < ZI; i++) {
                     const int o = 16 * (NW / ZN) * i;
 #pragma unroll
-                    for (int v = 0; v < 4; v++) x[i][v] = cur[(xq ^ (4 * v)) + o];
+                    for (int v = 0; v < 4; v++) x[i][v] = xi[v] >= 0 ? cur[xi[v] + o] : 0.0;
 #pragma unroll
                     for (int k = 1; k < KS; k++)
 #pragma unroll
@@ -373,11 +367,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                             z[i][v] += zs[((k - 1) * ZT + item) * 256 + v * 64 + lq];
 #pragma unroll
                     for (int v = 0; v < 4; v++) x[i][v] -= z[i][v];
-                    blocks(x[i], o, SEQ ? smask & 15 : smask | smask >> 4);
-                    if (lv && !(SEQ && gl == 1)) {
+                    blocks(x[i], SEQ ? smask & 15 : smask | smask >> 4);
 #pragma unroll
-                        for (int v = 0; v < 4; v++) cur[(xq ^ (4 * v)) + o] = x[i][v];
-                    }
+                    for (int v = 0; v < 4; v++)
+                        if (xi[v] >= 0 && !(SEQ && v >= gsplit)) cur[xi[v] + o] = x[i][v];
                 }
             }
             if constexpr (SEQ) {
@@ -392,15 +385,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                             const double av =
                                 cur[tpos<TS>(cfin + min(4 * b + (lq >> 4), a.g[0].w - 1), 16 * zm0 + liq) + o];
                             const double sv = sfl[64 * b + lq];
-                            y = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sv, y, 0, 0, 0);
+                            y = __builtin_amdgcn_mfma_f64_16x16x4f64(sv, av, y, 0, 0, 0);
                         }
 #pragma unroll
                         for (int v = 0; v < 4; v++) x[i][v] -= y[v];
-                        blocks(x[i], o, smask >> 4);
-                        if (lv && gl == 1) {
+                        blocks(x[i], smask >> 4);
 #pragma unroll
-                            for (int v = 0; v < 4; v++) cur[(xq ^ (4 * v)) + o] = x[i][v];
-                        }
+                        for (int v = 0; v < 4; v++)
+                            if (xi[v] >= 0 && v >= gsplit) cur[xi[v] + o] = x[i][v];
                     }
                 }
             }
