@@ -355,6 +355,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             };
             dbl4 x[ZI];
             if (solver) {
+                __builtin_amdgcn_s_setprio(3);
 #pragma unroll
                 for (int i = 0; i < ZI; i++) {
                     const int o = 16 * (NW / ZN) * i;
@@ -373,6 +374,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                         if (xi[v] >= 0 && !(SEQ && v >= gsplit)) cur[xi[v] + o] = x[i][v];
                 }
             }
+            if (solver) __builtin_amdgcn_s_setprio(0);
             if constexpr (SEQ) {
                 tp_barrier();
                 if (solver && a.ngrp == 2 && 16 * zn + 16 > a.g[1].zoff) {
