@@ -632,13 +632,16 @@ class Run {
             pa.lpb = lp_from_ >= 0 ? (int)(lp_from_ - cb) : (1 << 30);
         }
         int mt = 0, nbt = 0;
-        const int td = mx_ && !getenv("ORTH_MIXED_PASS32")
+        // FP64 products run on the FP64 passes.
+        const bool red = mx_ != 0 && mx_ != kMxFP64;
+        const int td = red && !getenv("ORTH_MIXED_PASS32")
                            ? pass16d_plan(pa, &mt, &nbt, lp_first_pass())
                            : 0;
         int64_t unit = kPassRows;
         int tsm = 0;
-        if (!mx_) {
+        if (!red) {
             unit = pass_rows(S_, pa);
+            if (unit == 0) return nullptr;
         } else if (td == 0) {
             // The 512-thread pass with super-tiles when the slab allows it,
             // else the 32-row mixed pass.
@@ -648,10 +651,6 @@ class Run {
             else if (pass16m_lds_bytes(pa) == 0)
                 return nullptr;
         }
-        // Workgroups per CU: the mixed pass with reduced-precision products
-        // runs one (its operand conversions need two waves' worth of
-        // registers), with FP64 products two, except the double-buffered one
-        // with 16 waves, which holds a whole CU.
         // One k_reduce_small launch after the pass sums its partials and runs
         // the small step.  ORTH_IN_PASS_SYNC=1 sums them in the pass's last
         // workgroups instead and launches only the small step after it, which
@@ -663,9 +662,9 @@ class Run {
         // The in-pass group sums follow the partials in `part`.
         bool tail = na > 0 && sc_.tickets && in_pass_sync_ && getenv("ORTH_IN_PASS_SYNC") &&
                     !getenv("ORTH_SEPARATE_REDUCE") && !getenv("ORTH_REDUCE_LAUNCH");
-        const int per_cu = !mx_                          ? pass_wg_per_cu(S_, pa)
-                           : td != 16 && mx_ == kMxFP64 ? 2
-                                                        : 1;
+        // A reduced-precision pass runs one workgroup per CU (its operand
+        // conversions need two waves' worth of registers).
+        const int per_cu = red ? 1 : pass_wg_per_cu(S_, pa, tail);
         int nwg = std::max(1, (int)(std::max(1, c_.ncu) * per_cu * wg_scale_));
         if (na > 0 && sc_.fixed) {
             // Fixed scratch: fewer row chunks, so that the partials fit.
@@ -701,7 +700,7 @@ class Run {
             wcols += pend_.g[g].w;
         }
         if (!timed(c_, ORTH_K_PASS, st_, flops, 8.0 * m_ * (ncols + wcols), [&] {
-                if (!mx_) return launch_pass(S_, pa, nwg, st_);
+                if (!red) return launch_pass(S_, pa, nwg, st_);
                 if (td > 0) return launch_pass16d_mixed(pa, mx_, td, nbt, nwg, st_);
                 return tsm > 0 ? launch_pass16bm(pa, mx_, nwg, st_)
                                : launch_pass16m(pa, mx_, nwg, st_);

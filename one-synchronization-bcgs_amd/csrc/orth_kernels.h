@@ -204,13 +204,12 @@ struct PassArgs {
     TailArgs tail;
 };
 
-// The FP64 passes (orth_pass.hip): does a call with n columns of block width
-// S fit them; rows per tile (the unit of a row chunk) and workgroups per CU
-// for a; launch.
+// The FP64 passes (orth_pass.hip): rows per tile (the unit of a row chunk)
+// and workgroups per CU for a (tail: the pass sums its own partials, which
+// takes no more LDS); launch.
 constexpr int kPassRows = 32;  // rows per tile of the mixed form
-bool pass_fits(int S, int64_t n);
 int pass_rows(int S, const PassArgs &a);
-int pass_wg_per_cu(int S, const PassArgs &a);
+int pass_wg_per_cu(int S, const PassArgs &a, bool tail);
 hipError_t launch_pass(int S, const PassArgs &a, int nwg, hipStream_t st);
 
 // The tile pass (orth_tpass.h) for S <= 16 and the wide-block pass
@@ -220,10 +219,16 @@ int tpass_rows(int S, const PassArgs &a);
 int tpass_wg_per_cu(int S, const PassArgs &a);
 hipError_t launch_tpass(int S, const PassArgs &a, int nwg, hipStream_t st);
 constexpr int kWpassMaxCols = 512;
-// Its coefficients: entry (k, n) of C (64 columns), in the order its lanes
+// Does a call with n columns of block width S run fused?  The tile pass takes
+// kTpassMaxCols columns with one 16-column tile of Z (S <= 8), 256 with two.
+inline bool pass_fits(int S, int64_t n)
+{
+    return n <= (S == kMaxS ? kWpassMaxCols : S == 16 ? 256 : kTpassMaxCols);
+}
+// The wide-block pass's coefficients: entry (k, n) of C (64 columns), in the order its lanes
 // hold them (one 16 x 16 tile: lane 16 (k % 4) + n % 16 holds rows k % 4 + 4 v).
 constexpr int kWpassN1 = 64;
-static inline __host__ __device__ int wpass_cidx(int k, int n)
+constexpr int wpass_cidx(int k, int n)
 {
     return (k >> 4) * (16 * kWpassN1) + (n >> 4) * 256 + ((k & 3) * 16 + (n & 15)) * 4 + ((k >> 2) & 3);
 }
@@ -231,23 +236,22 @@ int wpass_rows(int S, const PassArgs &a);
 int wpass_wg_per_cu(int S, const PassArgs &a);
 hipError_t launch_wpass(int S, const PassArgs &a, int nwg, hipStream_t st);
 
-// Mixed form with double-buffered direct-to-LDS loads in 32-row tiles
+// Reduced-precision mixed form with double-buffered direct-to-LDS loads in 32-row tiles
 // (rows_per must be a multiple of 32): waves per workgroup (8 or 16), or 0
 // when it does not apply.
 // any_width: also below the column bound (reduced precisions, whose
 // 512-thread pass runs one workgroup per CU).  min_cols: the column bound
 // (0: the library's default).
 int pass16d_plan(const PassArgs &a, int *mt, int *nb, bool any_width = false, int min_cols = 0);
-// Launch with the plan's waves per workgroup (nw) and N-tiles (nb): mx =
-// kMxFP64 (FP32 storage, FP64 products) or a reduced precision for the
-// projection tiles from lpb on.
+// Launch with the plan's waves per workgroup (nw) and N-tiles (nb): mx is
+// the reduced precision of the projection tiles from lpb on.
 hipError_t launch_pass16d_mixed(const PassArgs &a, int mx, int nw, int nb, int nwg,
                                 hipStream_t st);
 
 // Mixed-precision s = 16 pass (32-row tiles, 512 threads): mx selects the
-// reduced precision of the marked products (1 bf16, 2 fp16, 3 bf16x3 split,
-// 4 none: FP64 arithmetic on FP32-stored input).  pass16m_lds_bytes returns
-// 0 when the shape does not fit it.
+// reduced precision of the marked products (1 bf16, 2 fp16, 3 bf16x3 split);
+// pass16m_lds_bytes returns 0 when the shape does not fit it.  4, none (FP64
+// arithmetic on FP32-stored input), runs on the tile pass.
 enum { kMxBF16 = 1, kMxFP16 = 2, kMxBF16X3 = 3, kMxFP64 = 4 };
 // Host flag beside a reduced precision: only the first-pass projection and
 // Gram are reduced, the first-pass update stays FP64.

@@ -32,7 +32,7 @@ constexpr int kM = 512;    // threads per workgroup
 constexpr int kMPF = 16;   // prefetch registers per thread (32 rows x 256 columns)
 
 template <int NB, int MX>
-__global__ __launch_bounds__(kM) __attribute__((amdgpu_waves_per_eu(MX == kMxFP64 ? 4 : 2, MX == kMxFP64 ? 4 : 2))) void k_pass16m(PassArgs a)
+__global__ __launch_bounds__(kM) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_pass16m(PassArgs a)
 {
     constexpr int N1 = 32, TS = 32, LD = TS + 1, PSTEP = kM / TS;
     extern __shared__ double sm[];
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kM) __attribute__((amdgpu_waves_per_eu(MX == kMxFP6
     const bool proj = a.na > 0;
     bool lpt[NB];
 #pragma unroll
-    for (int tb = 0; tb < NB; tb++) lpt[tb] = MX != kMxFP64 && a.b0 + 16 * tb >= a.lpb;
+    for (int tb = 0; tb < NB; tb++) lpt[tb] = a.b0 + 16 * tb >= a.lpb;
     int acol[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) acol[j] = a.a0 + min(wave + 8 * j, max(Ma - 1, 0)) * 16 + li;
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kM) __attribute__((amdgpu_waves_per_eu(MX == kMxFP6
                 const int item = wave & 3, mt = item & 1, nt = item >> 1, kh = wave >> 2;
                 const bool mine = nks > 0 && (a.seq ? nt == (ORTH_G(a, p, zoff) >> 4)
                                                     : ztile_used(a, nt));
-                const bool zlp = MX != kMxFP64 && !a.seq && ztile_lp(a, nt);
+                const bool zlp = !a.seq && ztile_lp(a, nt);
                 dbl4 z = dbl4{0.0, 0.0, 0.0, 0.0};
                 if (mine) {
                     if (zlp) {
@@ -292,7 +292,6 @@ hipError_t launch_pass16m(const PassArgs &a, int mx, int nwg, hipStream_t st)
     case kMxBF16: return launch_pass16m_mx<kMxBF16>(a, lds, nwg, st);
     case kMxFP16: return launch_pass16m_mx<kMxFP16>(a, lds, nwg, st);
     case kMxBF16X3: return launch_pass16m_mx<kMxBF16X3>(a, lds, nwg, st);
-    case kMxFP64: return launch_pass16m_mx<kMxFP64>(a, lds, nwg, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -409,7 +408,6 @@ hipError_t launch_pass16bm(const PassArgs &a, int mx, int nwg, hipStream_t st)
     case kMxBF16: return launch_bm_mx<kMxBF16>(a, ts, mt, nb, lds, nwg, st);
     case kMxFP16: return launch_bm_mx<kMxFP16>(a, ts, mt, nb, lds, nwg, st);
     case kMxBF16X3: return launch_bm_mx<kMxBF16X3>(a, ts, mt, nb, lds, nwg, st);
-    case kMxFP64: return launch_bm_mx<kMxFP64>(a, ts, mt, nb, lds, nwg, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -501,7 +499,6 @@ hipError_t launch_pass16d_mixed(const PassArgs &a, int mx, int nw, int nb, int n
 {
     if ((nw != 8 && nw != 16) || a.rows_per % 32 != 0 || !a.X32) return hipErrorInvalidValue;
     switch (mx) {
-    case kMxFP64: return launch_pass16d_mx<kMxFP64>(a, nw, nb, nwg, st);
     case kMxBF16: return launch_pass16d_mx<kMxBF16>(a, nw, nb, nwg, st);
     case kMxFP16: return launch_pass16d_mx<kMxFP16>(a, nw, nb, nwg, st);
     case kMxBF16X3: return launch_pass16d_mx<kMxBF16X3>(a, nw, nb, nwg, st);

@@ -4,19 +4,12 @@
 
 namespace orth {
 
-bool pass_fits(int S, int64_t n)
-{
-    // Step 1 of the tile pass holds at most 256 columns of two-group
-    // coefficients; with two groups of at most 8 columns its buffers bound n.
-    return n <= (S == kMaxS ? kWpassMaxCols : S == 16 ? 256 : kTpassMaxCols);
-}
-
 int pass_rows(int S, const PassArgs &a)
 {
     return S == kMaxS ? wpass_rows(S, a) : tpass_rows(S, a);
 }
 
-int pass_wg_per_cu(int S, const PassArgs &a)
+int pass_wg_per_cu(int S, const PassArgs &a, bool)
 {
     return S == kMaxS ? wpass_wg_per_cu(S, a) : tpass_wg_per_cu(S, a);
 }

@@ -44,7 +44,7 @@ template <int MT, int NB, int F, bool EARLY, bool V2, int MX = 0>
 // Reduced-precision forms run one workgroup per CU (their operand
 // conversions need more than the 128 registers of two).
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
-    MX != 0 && MX != kMxFP64 ? 2 : 4, MX != 0 && MX != kMxFP64 ? 2 : 4))) void k_pass16b(PassArgs a)
+    MX != 0 ? 2 : 4, MX != 0 ? 2 : 4))) void k_pass16b(PassArgs a)
 {
     constexpr int N1 = 32, TS = 32 * F, LD = TS + 1;
     constexpr int LTS = F == 1 ? 5 : F == 2 ? 6 : F == 4 ? 7 : 8;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     // Mixed form: is this wave's Z tile (N-tile znt) a reduced-precision
     // product, and its coefficient chunks [zq0, zq0 + zqn) as MFMA B
     // fragments (lane: k = 8 lk + e of column li), converted once.
-    constexpr bool LP = MX != 0 && MX != kMxFP64;
+    constexpr bool LP = MX != 0;
     constexpr int MXL = LP ? MX : kMxBF16;  // operand format of the reduced-precision paths
     const int znt = F == 1 ? (wave >> 1) & 1 : wave & 1;
     const bool zlp = LP && !a.seq && ztile_lp(a, znt);

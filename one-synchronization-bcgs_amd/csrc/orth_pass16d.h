@@ -1,5 +1,5 @@
-// The FP64 fused pass for block width 16 with double-buffered direct-to-LDS
-// loads (32-row tiles; 512 threads and two workgroups per CU for slabs of at
+// The mixed form's fused pass with reduced-precision projections (block width
+// 16, double-buffered direct-to-LDS loads, 32-row tiles; 512 threads and two workgroups per CU for slabs of at
 // most 128 columns, 1024 threads and one workgroup per CU up to 256).
 //
 // Two LDS buffers hold consecutive tiles: right after the barrier that opens
@@ -83,20 +83,20 @@ __device__ __forceinline__ void lds_barrier()
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// MX = 0: the FP64 form.  MX != 0 (mixed form): columns from raw0 on (at
-// most 32, never step-1 operands) have not been written yet and come from the
-// FP32 input X32; they are loaded into registers together with the next
-// tile's DMA and written to LDS, widened, when that tile opens (a barrier
-// separates that write from their first reader).  With MX a reduced precision
-// (kMxBF16, kMxFP16, kMxBF16X3), the projection products whose B columns
-// start at or past lpb run as one 16 x 16 x 32 MFMA per 32-row tile with FP32
-// accumulation, summed across tiles in FP64; every other product is FP64.
+// MX: the reduced precision (kMxBF16, kMxFP16, kMxBF16X3).  Columns from raw0
+// on (at most 32, never step-1 operands) have not been written yet and come
+// from the FP32 input X32; they are loaded into registers together with the
+// next tile's DMA and written to LDS, widened, when that tile opens (a barrier
+// separates that write from their first reader).  The projection products
+// whose B columns start at or past lpb run as one 16 x 16 x 32 MFMA per 32-row
+// tile with FP32 accumulation, summed across tiles in FP64; every other
+// product is FP64.
 template <int NW, int NB, int MX>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_pass16d(
     PassArgs a)
 {
     constexpr int TS = 32, N1 = 32, kD = 64 * NW, LDc = kDLd;
-    constexpr bool MIX = MX != 0, LPP = MX != 0 && MX != kMxFP64;
+    constexpr bool MIX = MX != 0, LPP = MX != 0;
     constexpr int MXL = LPP ? MX : kMxBF16;  // operand format of the reduced-precision products
     // Step-1 work items: 2 x 2 Z tiles of 16 x 16, the inner dimension
     // split KS ways so that the items fill the NW waves.

@@ -26,7 +26,11 @@
 // the wave that sums a Z tile subtracts it from the columns of the groups
 // that own its 16 columns (two groups of at most 8 columns share one tile,
 // ZN = 1) and runs their blocked triangular solve on MFMA (one MFMA per
-// 4-column block with the row blocks [D_b | -D_b T] beside the factor); the
+// 4-column block with the row blocks [D_b | -D_b T] beside the factor), at
+// raised priority.  Z and the solve are transposed, so that a block's columns
+// are the next MFMA's operand as they stand; through LDS, at equal priority,
+// 2^20 x 256 (s = 16, A-1S) took 9.38 ms instead of 9.16, 2^24 x 256 135.6
+// instead of 130.4 (with a 13 ms copy).  The
 // groups go back to X; step 2 accumulates tile(:, a0:a0+na)^T
 // tile(:, b0:b0+nb), M-tile m by wave NW - 1 - m (mod NW), away from the
 // solving waves.
@@ -68,6 +72,7 @@ __device__ __forceinline__ int tpos(int c, int r)
 typedef __attribute__((address_space(3))) void tp_lds_t;
 typedef __attribute__((address_space(1))) const void tp_glb_t;
 typedef double dbl2t __attribute__((ext_vector_type(2)));
+typedef float flt4t __attribute__((ext_vector_type(4)));
 
 // A copy of v the optimizer cannot see through, so that addresses derived
 // from it inside the row loop are not hoisted into registers.
@@ -95,7 +100,11 @@ __device__ __forceinline__ void tp_wave_fence()
 // step 1 leaves those coefficient rows out, and the second group subtracts
 // their product after the first group's solve.
 // NW waves: 8 (two workgroups per CU) or 16 (one).  WIDE: over 256 columns.
-template <int NW, int TS, int NB, int ZN, int MT, bool WIDE, bool SEQ>
+// MIX: the mixed form with FP64 products.  Columns from raw0 on (at most 32,
+// never step-1 operands) have not been written yet and come from the FP32
+// input: a thread loads four rows of a column into registers beside the next
+// tile's LDS loads and widens them into the tile when it opens.
+template <int NW, int TS, int NB, int ZN, int MT, bool WIDE, bool SEQ, bool MIX = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_tpass(
     PassArgs a)
 {
@@ -215,12 +224,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     // moves four bytes per lane, a span in four loads.
     constexpr int CS = 128 / TS;  // columns per span
     const bool st16 = a.ldX % 2 == 0 && (uintptr_t)a.X % 16 == 0;
-    const int nspan = (a.ncols + CS - 1) / CS;
+    const int nspan = ((MIX ? min(a.ncols, a.raw0) : a.ncols) + CS - 1) / CS;
     const int lc0 = CS * wave + lane / (TS / 2), ls = lane & (TS / 2 - 1);
     const char *gb = (const char *)(a.X + rb + (int64_t)lc0 * a.ldX + 2 * (ls ^ tswz<TS>(lc0)));
     const int gx = TS == 128 ? 16 * ((ls ^ tswz<TS>(lc0 + NW)) - (ls ^ tswz<TS>(lc0))) : 0;
     const int64_t gs = (int64_t)CS * NW * a.ldX * 8;
-    const int ncols = a.ncols;
+    const int ncols = MIX ? min(a.ncols, a.raw0) : a.ncols;  // columns loaded into LDS
     auto issue = [&](int t, double *buf) {
         if (t >= nfull) return;
         const char *g = gb + (int64_t)t * (TS * 8);
@@ -246,6 +255,42 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 }
         }
     };
+    // Raw columns: chunk e = tid + kD q is rows 4 (e % (TS / 4)) .. + 3 of
+    // column ncols + e / (TS / 4); one 16-byte load where the input allows it.
+    constexpr int NRV = 8 * TS > kD ? 8 * TS / kD : 1;
+    const int nraw = a.ncols - ncols;
+    const bool rv4 = MIX && a.ldX32 % 4 == 0 && (uintptr_t)a.X32 % 16 == 0;
+    flt4t rv[MIX ? NRV : 1];
+    auto raw_load = [&](int t) {
+        if constexpr (MIX) {
+            if (t >= nfull) return;
+#pragma unroll
+            for (int q = 0; q < NRV; q++) {
+                const int e = tp_opaque(tid) + kD * q, c = e / (TS / 4);
+                if (c >= nraw) continue;
+                const float *p = a.X32 + rb + (int64_t)t * TS + 4 * (e % (TS / 4)) +
+                                 (int64_t)(ncols + c) * a.ldX32;
+                if (rv4) {
+                    rv[q] = __builtin_nontemporal_load((const flt4t *)p);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) rv[q][k] = __builtin_nontemporal_load(p + k);
+                }
+            }
+        }
+    };
+    auto raw_store = [&](double *buf) {
+        if constexpr (MIX) {
+#pragma unroll
+            for (int q = 0; q < NRV; q++) {
+                const int e = tp_opaque(tid) + kD * q, c = e / (TS / 4), r = 4 * (e % (TS / 4));
+                if (c >= nraw) continue;
+                *(dbl2t *)(buf + tpos<TS>(ncols + c, r)) = dbl2t{(double)rv[q][0], (double)rv[q][1]};
+                *(dbl2t *)(buf + tpos<TS>(ncols + c, r + 2)) = dbl2t{(double)rv[q][2], (double)rv[q][3]};
+            }
+        }
+    };
+    raw_load(0);
     issue(0, sm);
 
     // Write-back: LP threads per column, row pairs sq + LP i.
@@ -277,15 +322,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
         else
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const int lq = tp_opaque(lane), liq = lq & 15;
+        if (MIX && t < nfull) raw_store(cur);
         if (t >= nfull) {
             // The matrix's last rows: element by element, zeros past them.
             const int64_t r0 = rb + (int64_t)t * TS;
-            for (int e = tp_opaque(tid); e < ncols * TS; e += kD) {
+            for (int e = tp_opaque(tid); e < a.ncols * TS; e += kD) {
                 const int c = e / TS, r = e % TS;
-                cur[tpos<TS>(c, r)] = r0 + r < re ? a.X[r0 + r + (int64_t)c * a.ldX] : 0.0;
+                double x = 0.0;
+                if (r0 + r < re)
+                    x = MIX && c >= ncols ? (double)a.X32[r0 + r + (int64_t)c * a.ldX32]
+                                          : a.X[r0 + r + (int64_t)c * a.ldX];
+                cur[tpos<TS>(c, r)] = x;
             }
             tp_barrier();
+        } else if (MIX && !hasg) {
+            tp_barrier();  // (with groups the raw columns' readers wait in step 1)
         }
+        if (MIX) raw_load(t + 1);
         if (!late) issue(t + 1, nxt);
 
         if (hasg) {

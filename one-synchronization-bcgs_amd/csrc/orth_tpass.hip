@@ -32,7 +32,9 @@ constexpr int64_t kTpCached = 256 << 20;  // bytes of the last-level cache
 TpPlan plan(int S, const PassArgs &a)
 {
     TpPlan p;
-    if (S > 16 || a.X32 || a.n1 > 32) return p;
+    if (S > 16 || a.n1 > 32) return p;
+    // Mixed form: at most 32 raw columns, none of them a step-1 operand.
+    if (a.X32 && (a.n1 != 32 || a.seq || a.raw0 < a.k1 || a.ncols - a.raw0 > 32)) return p;
     int wl = std::max(a.ncols, a.k1);
     if (a.na > 0) {
         const int Ma = (a.na + 15) / 16, Nb = (a.nb + 15) / 16;
@@ -69,18 +71,18 @@ size_t lds_t(int wl, int seq)
     return (size_t)(2 * wl * TS + TpZ<NW, TS, ZN, false>::Zs + (seq ? 256 : 0)) * sizeof(double);
 }
 
-template <int NW, int TS, int NB, int ZN, int MT, bool WIDE, bool SEQ>
+template <int NW, int TS, int NB, int ZN, int MT, bool WIDE, bool SEQ, bool MIX = false>
 hipError_t launch_t(const PassArgs &a, int nwg, hipStream_t st)
 {
     static bool attr_set = false;
     if (!attr_set) {
         hipError_t e =
-            hipFuncSetAttribute((const void *)k_tpass<NW, TS, NB, ZN, MT, WIDE, SEQ>,
+            hipFuncSetAttribute((const void *)k_tpass<NW, TS, NB, ZN, MT, WIDE, SEQ, MIX>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024));
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    k_tpass<NW, TS, NB, ZN, MT, WIDE, SEQ>
+    k_tpass<NW, TS, NB, ZN, MT, WIDE, SEQ, MIX>
         <<<dim3(nwg), dim3(64 * NW), lds_t<NW, TS, ZN>(a.wl, SEQ), st>>>(a);
     return hipGetLastError();
 }
@@ -88,6 +90,12 @@ hipError_t launch_t(const PassArgs &a, int nwg, hipStream_t st)
 template <int NW, int TS, int MT, bool WIDE, bool SEQ>
 hipError_t launch_n(const PassArgs &a, int nwg, hipStream_t st)
 {
+    if constexpr (!WIDE && !SEQ) {
+        if (a.X32)
+            return a.nb > 16 ? launch_t<NW, TS, 2, 2, MT, false, false, true>(a, nwg, st)
+                             : launch_t<NW, TS, 1, 2, MT, false, false, true>(a, nwg, st);
+    }
+    if (a.X32) return hipErrorInvalidValue;
     if (a.n1 <= 16) return launch_t<NW, TS, 1, 1, MT, WIDE, SEQ>(a, nwg, st);
     return a.nb > 16 ? launch_t<NW, TS, 2, 2, MT, WIDE, SEQ>(a, nwg, st)
                      : launch_t<NW, TS, 1, 2, MT, WIDE, SEQ>(a, nwg, st);

@@ -17,7 +17,11 @@
 // wave of the first one (slice 0) collects both, subtracts them and runs the
 // blocked triangular solve (8 blocks of 4 columns, one MFMA per block and
 // tile), while the other waves issue the next tile's loads and start on the
-// part of the projection that no group takes part in.
+// part of the projection that no group takes part in.  Z and the solve are
+// transposed, as in the tile pass.
+//
+// 2^22 x 512, s = 32, P-1S: 110 ms (F = 4 m n^2 at 40 TFLOP/s) where separate
+// projection and update kernels took 178.
 #pragma once
 
 #include "orth_tpass.h"
