@@ -107,8 +107,8 @@ int orth_bcgs_mixed_device(int variant, int precision, int64_t m, int64_t n,
  * m[i] x n[i] with block width s[i], device dX[i] (ld ldX[i]) becomes Q,
  * device dR[i] (ld ldR[i]) receives R).  Instances run side by side on
  * several internal streams, each with private scratch; the batch is
- * captured into hipGraphs and replayed while the same batch (shapes and
- * pointers) is passed again.  tune != 0 first times the stream count and
+ * captured into hipGraphs, at its second call in a row or after tuning, and
+ * replayed while the same batch (shapes and pointers) is passed again.  tune != 0 first times the stream count and
  * workgroup share on this batch and keeps the best for batches with the
  * same shapes; it also decides between replaying captured graphs and
  * launching directly on the streams, and picks the tile shape of the s = 16
