@@ -164,6 +164,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
     }
     early = __builtin_amdgcn_readfirstlane(early);
+    // One slice: are columns of a group's second Z tile step-1 operands (the
+    // folded form's second group multiplies the first group's columns)?  Then
+    // a barrier separates step 1 from the subtraction in place (a slot in LDS
+    // does not fit beside two full buffers and two groups' solve operands).
+    bool hand = false;
+    if (KS == 1)
+        for (int g = 0; g < a.ngrp; g++)
+            hand = hand || (ORTH_G(a, g, w) > 16 && ORTH_G(a, g, t0) + 16 < a.k1);
 
     const int64_t rb = (int64_t)blockIdx.x * a.rows_per;
     const int64_t re = min(a.m, rb + a.rows_per);
@@ -333,7 +341,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             if (NW == 8) __builtin_amdgcn_s_setprio(0);
             // Hand the Z tiles to the collecting waves: partials through LDS,
-            // or (one slice) a group's second tile by subtracting it in place.
+            // or (one slice) a group's second tile by subtracting it in place,
+            // after every wave's last read of those columns (hand).
+            if (KS == 1 && hand) tp_barrier();
             if constexpr (KS > 1) {
                 if (ksp > 0 || half == 1) {
                     const int slot = ksp > 0 ? (ksp - 1) * ZN + zn : (KS - 1) * ZN + gi;
