@@ -11,6 +11,8 @@ namespace orth {
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ bool is_nan(double x) { return __builtin_amdgcn_class(x, 0x3); }
+
 // Group fields by a runtime index without indexing the kernel-argument
 // array (which would force a private copy of the arguments).
 #define ORTH_G(args_, idx_, fld_) ((idx_) == 0 ? (args_).g[0].fld_ : (args_).g[1].fld_)

@@ -18,9 +18,20 @@ constexpr int kLdT = 32;   // leading dimension of every s x s factor
 // kSlotW + 128 b) holds D_b = inv(T(4b:4b+4, 4b:4b+4)) in columns 4b..4b+3,
 // -D_b T(4b:4b+4, c) in the columns c right of the block, zero elsewhere and
 // past the factor's width.  All are written by the Cholesky step.
+// After a pivot that is not positive, the row blocks solve for the columns
+// before it only: they are zero in its row and column and past them, except
+// that column c is NaN in block slot_last(c, w), the last one the solve takes
+// for it.  A pass that also takes zeros for those columns of X, whose entries
+// need not be finite, leaves NaN there and the columns before them intact, as
+// the row-wise solve does.
 constexpr int kSlotRecip = kLdT * kLdT;
 constexpr int kSlotW = kSlotRecip + kLdT;
 constexpr int kSlot = kSlotW + (kMaxS / 4) * 4 * kLdT;
+constexpr int slot_last(int c, int w)
+{
+    const int o = (w - 1) & ~3, e = c < 16 ? 12 : 28;
+    return o < e ? o : e;
+}
 
 // One row-local block update of a streaming pass:
 //   X(:, col0:col0+w) <- (X(:, col0:col0+w) - X(:, 0:c) * W) * T^{-1}

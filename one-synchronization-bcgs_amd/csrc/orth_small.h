@@ -251,9 +251,11 @@ static __device__ __forceinline__ void wave_solve_z2(int w0, int w1, const doubl
 // and the row blocks of the blocked solve, whose row D_b(k, :) of the
 // inverted 4 x 4 diagonal block each thread forms for itself:
 // D(k,k) = 1/u(k,k), D(k,j) = -(sum_{i=k}^{j-1} D(k,i) u(i,j)) / u(j,j).
-// Entries past W keep the zeros the call started with.
+// Entries past W keep the zeros the call started with.  p: the first bad pivot
+// (w: none); the row blocks then solve for the columns before it and leave NaN
+// in the others (see orth_kernels.h).
 template <int W>
-static __device__ __forceinline__ void d_write_slot(int t, int n, int w, const double *M,
+static __device__ __forceinline__ void d_write_slot(int t, int n, int w, int p, const double *M,
                                                     const double *rc, double *T)
 {
     constexpr int L = SmallLay<W>::L, LW = SmallLay<W>::LW;
@@ -274,6 +276,8 @@ static __device__ __forceinline__ void d_write_slot(int t, int n, int w, const d
 #pragma unroll
         for (int j = 0; j < 4; j++)
             v = c >= o + 4 ? (o + j < w ? fma(-d[j], M[(o + j) * L + c], v) : v) : c == o + j ? d[j] : v;
+        if (p < w && (i >= p || c >= p))
+            v = c >= p && o == slot_last(c, w) ? __builtin_nan("") : 0.0;
         T[kSlotW + o * kLdT + (i & 3) * kLdT + c] = in ? v : 0.0;
     }
 }
@@ -481,7 +485,7 @@ static __device__ __forceinline__ void small_step(int nt, const SmallArgs &a, do
         wave_solve_z2<W>(wb, wn, M, Z);
     } else if (wave >= 2) {
         const int t = tid - 128, n = nt - 128;
-        d_write_slot<W>(t, n, wb, M, rc, qr ? a.Cq + (op - OP_CQR1) * kSlot : close ? a.Om : a.Sig);
+        d_write_slot<W>(t, n, wb, info[0] > 0 ? info[0] - 1 : wb, M, rc, qr ? a.Cq + (op - OP_CQR1) * kSlot : close ? a.Om : a.Sig);
         // R_bb = Omega Sigma (Omega in the A-1S form); S_bot to R and P.
         if (close) {
             if (mode == 2) d_trmm<W>(t, n, wb, M, L, a.Sig, Rb + c, 1, a.ldR);
@@ -514,7 +518,7 @@ static __device__ __forceinline__ void small_step(int nt, const SmallArgs &a, do
     if (pyth || fold) __syncthreads();
     if (pyth) {
         if (tid == 0) note_info(a.status, a.blk + 1, info[1]);
-        d_write_slot<W>(tid, nt, wn, M + W * L + W, rc + W, a.Sig);
+        d_write_slot<W>(tid, nt, wn, info[1] > 0 ? info[1] - 1 : wn, M + W * L + W, rc + W, a.Sig);
     }
     if (a.Cout) {
         // Next pass: the first group finalizes block b with [Y; 0] (closing

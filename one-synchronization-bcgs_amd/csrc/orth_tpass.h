@@ -97,8 +97,8 @@ __device__ __forceinline__ void tp_wave_fence()
 }
 
 // SEQ: the second group's product uses the first group's finished columns:
-// step 1 leaves those coefficient rows out, and the second group subtracts
-// their product after the first group's solve.
+// step 1 ends before them, and the second group subtracts their product after
+// the first group's solve.
 // NW waves: 8 (two workgroups per CU) or 16 (one).  WIDE: over 256 columns.
 // MIX: the mixed form with FP64 products.  Columns from raw0 on (at most 32,
 // never step-1 operands) have not been written yet and come from the FP32
@@ -133,7 +133,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const int item = wave % ZT, ksp = wave / ZT;
     const int zn = item % ZN, zm0 = item / ZN;
     const bool zany = ztile_used(a, zn);
-    const int nu = zany ? (a.k1 + 15) >> 4 : 0;
+    const int cfin = SEQ ? a.g[0].t0 : 0;  // first finished column of the sequential form
+    const int k1 = SEQ ? min(a.k1, cfin) : a.k1;
+    const int nu = zany ? (k1 + 15) >> 4 : 0;
     const int ulo = nu * ksp / KS, nun = nu * (ksp + 1) / KS - ulo;
     const int uf = ulo + nun == nu ? nu - 1 : ulo;  // the first unit taken
     const int ur = uf == ulo ? ulo + 1 : ulo;       // start of the others
@@ -142,21 +144,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const int gl = a.ngrp == 2 && zc >= a.g[1].zoff ? 1 : 0;
     const int goff = zc - ORTH_G(a, gl, zoff);
     const bool lv = gl < a.ngrp && goff >= 0 && goff < ORTH_G(a, gl, w);
-    const int cfin = SEQ ? a.g[0].t0 : 0;  // first finished column of the sequential form
     double cf[UQ][4];
 #pragma unroll
     for (int u = 0; u < UQ; u++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int k = 16 * (u == 0 ? uf : ur + u - 1) + 4 * v + lk;
-            const bool in = u < nun && k < a.k1 && !(SEQ && gl == 1 && k >= cfin);
-            cf[u][v] = in ? a.C[k * N1 + zc] : 0.0;
+            cf[u][v] = u < nun && k < k1 ? a.C[k * N1 + zc] : 0.0;
         }
     // Index of k-step 0 of units uf and ur; k-step v is this XOR 4 v, plus
     // 4 v TS.
     const int zf = tpos<TS>(16 * uf + lk, 16 * zm0 + li);
     const int zr = tpos<TS>(16 * ur + lk, 16 * zm0 + li);
-    const int kc = 16 * uf + 16 > a.k1 ? a.k1 - 1 : 1 << 20;  // column clamp of unit uf
+    const int kc = 16 * uf + 16 > k1 ? k1 - 1 : 1 << 20;  // column clamp of unit uf
     // The Z tile is computed transposed (lane: row li of the chunk, columns
     // lk + 4 v), so that value v of the chunk is the operand of block v of the
     // blocked solve.  xi: the index of column lk + 4 v, or -1 past its group.
@@ -198,6 +198,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
         for (int v = 0; v < 4; v++) asm volatile("" ::"v"(cf[u][v]));
 #pragma unroll
     for (int b = 0; b < 4; b++) asm volatile("" ::"v"(bw[b]));
+    // Z columns past a bad pivot (bit), which the solve must not see.
+    const uint32_t badc = (uint32_t)__ballot(is_nan(bw[0]) | is_nan(bw[1]) | is_nan(bw[2]) |
+                                             is_nan(bw[3])) & 0xffff;
 
     // Projection: M-tiles m0 + NW i, all NB N-tiles.  Operand of k-step ks:
     // row 4 ks + lk, i.e. the base index XOR 4 (ks & 7), plus 32 (ks >> 3).
@@ -391,6 +394,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             // the partial Z tiles; then the blocked triangular solve, whose
             // chain is its MFMAs alone.
             auto blocks = [&](dbl4 &x, int mask) {
+                if (badc) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        if (badc >> (4 * v + (lq >> 4)) & 1) x[v] = 0.0;
+                }
 #pragma unroll
                 for (int b = 0; b < 4; b++) {
                     if (!(mask >> b & 1)) continue;

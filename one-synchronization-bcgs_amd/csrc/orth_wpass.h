@@ -79,11 +79,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const bool zany = 16 * half < gw;
     const int zc = 16 * zn + li;
     const int cfin = SEQ ? a.g[0].t0 : 0;  // first finished column of the sequential form
-    const int klim = SEQ && gi == 1 ? min(cfin, a.k1) : a.k1;  // rows of C this tile uses
+    const int k1 = SEQ ? min(cfin, a.k1) : a.k1;
     // Units [ulo, ulo + nun) of 16 columns.  The slice that holds the last
     // unit, which may reach past k1, takes it first, from column addresses
     // clamped below k1 (zero coefficients).
-    const int nu = zany ? (a.k1 + 15) >> 4 : 0;
+    const int nu = zany ? (k1 + 15) >> 4 : 0;
     const int ulo = nu * ksp / KS, nun = nu * (ksp + 1) / KS - ulo;
     const int uf = ulo + nun == nu ? nu - 1 : ulo;  // the first unit taken
     const int ur = uf == ulo ? ulo + 1 : ulo;       // start of the others
@@ -93,9 +93,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int k = 16 * (u == 0 ? uf : ur + u - 1) + 4 * v + lk;
-            cf[u][v] = u < nun && k < klim ? a.C[wpass_cidx(k, zc)] : 0.0;
+            cf[u][v] = u < nun && k < k1 ? a.C[wpass_cidx(k, zc)] : 0.0;
         }
-    const int kc = 16 * uf + 16 > a.k1 ? a.k1 - 1 : 1 << 20;  // column clamp of unit uf
+    const int kc = 16 * uf + 16 > k1 ? k1 - 1 : 1 << 20;  // column clamp of unit uf
     // Units UR .. nun - 1 are whole ones, from L2: the first at row ks0 of C.
     const int nst = max(nun - UR, 0);
     const int ks0 = 16 * (ur + UR - 1);
@@ -107,6 +107,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const double *T = ORTH_G(a, g, T);
         if (T)
             for (int e = tid; e < 1024; e += kD) wf[1024 * g + e] = T[kSlotW + e];
+    }
+    // Good columns of this wave's group: those before a bad pivot.
+    int gx = gw;
+    if (gT && solver) {
+        const int c = lane & (kLdT - 1);
+        const uint32_t bad = (uint32_t)__ballot(
+            c < gw && is_nan(gT[kSlotW + slot_last(c, gw) * kLdT + c]));
+        if (bad) gx = __builtin_ctz(bad);
     }
     // Sequential form: the second group's coefficients on the first group's
     // columns.
@@ -171,7 +179,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     bool hand = false;
     if (KS == 1)
         for (int g = 0; g < a.ngrp; g++)
-            hand = hand || (ORTH_G(a, g, w) > 16 && ORTH_G(a, g, t0) + 16 < a.k1);
+            hand = hand || (ORTH_G(a, g, w) > 16 && ORTH_G(a, g, t0) + 16 < k1);
 
     const int64_t rb = (int64_t)blockIdx.x * a.rows_per;
     const int64_t re = min(a.m, rb + a.rows_per);
@@ -262,11 +270,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 const char *cu = (const char *)(a.C + k * N1 + 256 * zn) + cl;
                 const dbl2t x = ((const dbl2t *)cu)[0], y = ((const dbl2t *)cu)[1];
                 c[0] = x.x, c[1] = x.y, c[2] = y.x, c[3] = y.y;
-                if constexpr (SEQ) {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        if (k + 4 * v + lkq >= klim) c[v] = 0.0;
-                }
             };
             if (US > 0 && nst > 0) {
                 cload(c0, 0);
@@ -420,13 +423,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         }
                     }
                 }
-                // Columns past the group: zero, with zero rows of W.
+                // Columns past the good ones: zero, with zero rows of W.
 #pragma unroll
                 for (int i = 0; i < ZI; i++)
 #pragma unroll
                     for (int v = 0; v < 4; v++) {
-                        if (4 * v + lkq >= gw) x0[i][v] = 0.0;
-                        if (16 + 4 * v + lkq >= gw) x1[i][v] = 0.0;
+                        if (4 * v + lkq >= gx) x0[i][v] = 0.0;
+                        if (16 + 4 * v + lkq >= gx) x1[i][v] = 0.0;
                     }
                 if (gT) {
                     // (Rows of W past the group are zero.)

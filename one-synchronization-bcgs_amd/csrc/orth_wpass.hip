@@ -112,6 +112,8 @@ hipError_t launch_wpass(int S, const PassArgs &a0, int nwg, hipStream_t st)
     PassArgs a = a0;
     a.wl = p.wl;
     a.bsh = p.bsh;
+    // The sequential form's last block: its own columns are no operands.
+    if (a.seq && a.ngrp == 1) a.k1 = std::min(a.k1, a.g[0].t0);
     if (p.nw == 8) return launch_n<8, 16, 4>(a, p, nwg, st);
     switch (p.ts) {
     case 16: return launch_n<4, 16, 4>(a, p, nwg, st);
