@@ -164,7 +164,9 @@ static __device__ __forceinline__ void wave_syrk(int k, int r0, int nr, int c0, 
 // right-looking elimination, a lane keeps every RG-th row of one column in
 // registers, the pivot row goes through LDS, and the only division on the
 // chain is the pivot's reciprocal (the square roots scale the rows at the
-// end).  A pivot that is not positive makes everything after it NaN.
+// end); a pivot whose reciprocal would leave the normal range goes through its
+// square root instead.  A pivot that is not positive makes everything after
+// it NaN.
 // *info: 0 or the 1-based first such pivot.
 template <int W>
 static __device__ __forceinline__ void wave_chol(int w, int nc, double *M, double *rc, int *info)
@@ -191,10 +193,14 @@ static __device__ __forceinline__ void wave_chol(int w, int nc, double *M, doubl
             for (int q = 0; q < NQ; q++) a[q] = Mk[b0 + RG * q + h];
             const bool good = d > 0.0;
             if (!good && bad == 0) bad = b0 + k + 1;
-            const double r = good ? 1.0 / d : __builtin_nan("");
+            double r = good ? 1.0 / d : __builtin_nan(""), x = mk;
+            if (good && !(d >= 0x1p-1000 && d <= 0x1p1000)) {
+                r = 1.0 / sqrt(d);
+                x = mk * r;
+            }
 #pragma unroll
             for (int q = 0; q < NQ; q++)
-                if (RG * q + h > k) m[q] = fma(-(a[q] * r), mk, m[q]);
+                if (RG * q + h > k) m[q] = fma(-(a[q] * r), x, m[q]);
 #pragma unroll
             for (int q = 0; q < NQ; q++)
                 if (act && RG * q + h < wb) Mb[(RG * q + h) * L + j] = m[q];
