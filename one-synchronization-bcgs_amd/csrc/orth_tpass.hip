@@ -45,7 +45,9 @@ TpPlan plan(int S, const PassArgs &a)
         p.bsh = std::max(0, a.b0 + 16 * Nb - wl);
     }
     wl = (wl + 15) / 16 * 16;
-    if (wl > kTpassMaxCols) return p;
+    // A projection on a block at the slab's end (the intra-block QR) pads its
+    // M-tile past the last column.
+    if (a.ncols > kTpassMaxCols || wl > kTpassMaxCols + 16) return p;
     for (int g = 0; g < a.ngrp; g++)
         if (a.g[g].t0 + a.g[g].w > a.ncols || a.g[g].zoff % 4 != 0 ||
             a.g[g].zoff / 16 != (a.g[g].zoff + a.g[g].w - 1) / 16)
