@@ -169,8 +169,9 @@ bool is_device_ptr(const void *p)
     return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
 }
 
-// Can a kernel on the current device write to p?  (Pinned host memory is
-// mapped; another device's memory and pageable memory go through copies.)
+// Can a kernel on the current device write to p?  Pinned host memory is mapped
+// at its own address; registered host memory may be mapped at another one, and
+// goes through copies like another device's memory and pageable memory.
 bool kernel_writable(const void *p)
 {
     hipPointerAttribute_t at;
@@ -180,7 +181,8 @@ bool kernel_writable(const void *p)
         return false;
     }
     if (at.type == hipMemoryTypeDevice) return at.device == current_device();
-    return at.type == hipMemoryTypeManaged || at.type == hipMemoryTypeHost;
+    if (at.type == hipMemoryTypeHost) return at.devicePointer == p;
+    return at.type == hipMemoryTypeManaged;
 }
 
 // Records start/stop events around one launch when timing is enabled.
