@@ -1404,23 +1404,37 @@ bool batch_capture(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg)
 // replays the graphs captured for this exact batch; a batch met for the
 // first time is launched directly on the streams (which also makes every
 // kernel's first launch, and its launch attributes, happen outside capture).
-// A direct run is followed by a capture, without running, for the next call
-// when the call before was for the same batch too, or with `capture` at once:
-// a caller with new buffers in every call would pay for graphs it never
-// replays (48 uneven instances of 2^12 to 2^18 rows: 9.6 ms a call, 16.0 with
-// a capture in each).
+// When the next call is for the same batch, it is captured and the graphs are
+// replayed at once; with `capture` the first run is followed by the capture.
+// Not every first run: a caller with new buffers in every call would pay for
+// graphs it never replays.  48 uneven instances of 2^12 to 2^18 rows: first
+// call 12.7 ms, second 11.0 (13.8 as a direct run followed by the capture),
+// the others 8.7.
 bool batch_run(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg, bool capture)
 {
     const std::vector<int64_t> key = full_key(a, cfg);
-    if (cfg.graph && !b.execs.empty() && key == b.key) {
+    auto replay = [&] {
         for (hipGraphExec_t e : b.execs)
             if (!ok(hipGraphLaunch(e, b.main))) return false;
         return ok(hipStreamSynchronize(b.main));
-    }
-    capture = capture || key == b.seen;
-    b.seen = key;
+    };
+    // Capture for this key; a batch that cannot be captured is launched
+    // directly from now on.
+    auto take = [&] {
+        if (batch_capture(b, a, cfg))
+            b.key = key;
+        else
+            b.nocap = key;
+        return !b.broken;
+    };
+    if (cfg.graph && !b.execs.empty() && key == b.key) return replay();
     drop_graphs(b);
     if (!batch_reserve(b, a, cfg.streams)) return false;
+    if (cfg.graph && key == b.seen && key != b.nocap) {
+        if (!take()) return false;
+        if (!b.execs.empty()) return replay();
+    }
+    b.seen.clear();
     std::vector<int> all(a.count);
     for (int i = 0; i < a.count; i++) all[i] = i;
     freeze(b, true);
@@ -1428,15 +1442,8 @@ bool batch_run(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg, bool captur
     freeze(b, false);
     const bool done = ok(hipStreamSynchronize(b.main));
     if (!enq || !done) return false;
-    if (cfg.graph && capture && key != b.nocap) {
-        if (batch_capture(b, a, cfg))
-            b.key = key;
-        else if (b.broken)
-            return false;
-        else
-            b.nocap = key;  // launched directly from now on
-    }
-    return true;
+    b.seen = key;
+    return cfg.graph && capture && key != b.nocap ? take() : true;
 }
 
 // Device copies of the batch's FP64 inputs, so that every timing run of the
