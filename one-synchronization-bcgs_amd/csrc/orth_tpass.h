@@ -394,11 +394,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             // the partial Z tiles; then the blocked triangular solve, whose
             // chain is its MFMAs alone.
             auto blocks = [&](dbl4 &x, int mask) {
-                if (badc) {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        if (badc >> (4 * v + (lq >> 4)) & 1) x[v] = 0.0;
-                }
 #pragma unroll
                 for (int b = 0; b < 4; b++) {
                     if (!(mask >> b & 1)) continue;
@@ -415,6 +410,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 }
             };
             dbl4 x[ZI];
+            auto contain = [&] {
+                if (badc) {
+#pragma unroll
+                    for (int i = 0; i < ZI; i++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++)
+                            if (badc >> (4 * v + (lq >> 4)) & 1) x[i][v] = 0.0;
+                }
+            };
             if (solver) {
                 __builtin_amdgcn_s_setprio(3);
 #pragma unroll
@@ -429,6 +433,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                             z[i][v] += zs[((k - 1) * ZT + item) * 256 + v * 64 + lq];
 #pragma unroll
                     for (int v = 0; v < 4; v++) x[i][v] -= z[i][v];
+                }
+                contain();
+#pragma unroll
+                for (int i = 0; i < ZI; i++) {
+                    const int o = 16 * (NW / ZN) * i;
                     blocks(x[i], SEQ ? smask & 15 : smask | smask >> 4);
 #pragma unroll
                     for (int v = 0; v < 4; v++)
@@ -452,6 +461,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                         }
 #pragma unroll
                         for (int v = 0; v < 4; v++) x[i][v] -= y[v];
+                    }
+                    contain();
+#pragma unroll
+                    for (int i = 0; i < ZI; i++) {
+                        const int o = 16 * (NW / ZN) * i;
                         blocks(x[i], smask >> 4);
 #pragma unroll
                         for (int v = 0; v < 4; v++)
