@@ -191,12 +191,17 @@ static __device__ __forceinline__ void wave_chol(int w, int nc, double *M, doubl
             double a[NQ];
 #pragma unroll
             for (int q = 0; q < NQ; q++) a[q] = Mk[b0 + RG * q + h];
-            const bool good = d > 0.0;
-            if (!good && bad == 0) bad = b0 + k + 1;
-            double r = good ? 1.0 / d : __builtin_nan(""), x = mk;
-            if (good && !(d >= 0x1p-1000 && d <= 0x1p1000)) {
-                r = 1.0 / sqrt(d);
-                x = mk * r;
+            double r = 1.0 / d, x = mk;
+            // One scalar comparison beside the chain: 2^-1000 <= d < 2^1000.
+            const uint32_t hi = __builtin_amdgcn_readfirstlane(__double2hiint(d));
+            if (__builtin_expect(hi - (23u << 20) >= 2000u << 20, 0)) {
+                if (d > 0.0) {
+                    r = 1.0 / sqrt(d);
+                    x = mk * r;
+                } else {
+                    r = __builtin_nan("");
+                    if (bad == 0) bad = b0 + k + 1;
+                }
             }
 #pragma unroll
             for (int q = 0; q < NQ; q++)
