@@ -189,6 +189,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             }
         }
     }
+    // Z columns past a bad pivot, which the solve must not see: bits 8 to 23 of
+    // smask (one scalar for both: the kernel has none to spare).
+    const bool badl = is_nan(bw[0]) || is_nan(bw[1]) || is_nan(bw[2]) || is_nan(bw[3]);
+    smask |= ((int)__ballot(badl) & 0xffff) << 8;
     smask = __builtin_amdgcn_readfirstlane(smask);
     const int gsplit = a.ngrp == 2 ? a.g[1].zoff / 4 - 4 * zn : 4;  // first block of group 1
     // Make the compiler wait for these loads here, once.
@@ -198,9 +202,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
         for (int v = 0; v < 4; v++) asm volatile("" ::"v"(cf[u][v]));
 #pragma unroll
     for (int b = 0; b < 4; b++) asm volatile("" ::"v"(bw[b]));
-    // Z columns past a bad pivot (bit), which the solve must not see.
-    const uint32_t badc = (uint32_t)__ballot(is_nan(bw[0]) | is_nan(bw[1]) | is_nan(bw[2]) |
-                                             is_nan(bw[3])) & 0xffff;
 
     // Projection: M-tiles m0 + NW i, all NB N-tiles.  Operand of k-step ks:
     // row 4 ks + lk, i.e. the base index XOR 4 (ks & 7), plus 32 (ks >> 3).
@@ -411,12 +412,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             };
             dbl4 x[ZI];
             auto contain = [&] {
-                if (badc) {
+                if (smask >> 8) {
 #pragma unroll
                     for (int i = 0; i < ZI; i++)
 #pragma unroll
                         for (int v = 0; v < 4; v++)
-                            if (badc >> (4 * v + (lq >> 4)) & 1) x[i][v] = 0.0;
+                            if (smask >> (8 + 4 * v + (lq >> 4)) & 1) x[i][v] = 0.0;
                 }
             };
             if (solver) {
