@@ -635,10 +635,9 @@ class Run {
         }
         int mt = 0, nbt = 0;
         // FP64 products run on the FP64 passes.
-        const bool red = mx_ != 0 && mx_ != kMxFP64;
-        const int td = red && !getenv("ORTH_MIXED_PASS32")
-                           ? pass16d_plan(pa, &mt, &nbt, lp_first_pass())
-                           : 0;
+        const bool red = lp_first_pass();
+        const int td =
+            red && !getenv("ORTH_MIXED_PASS32") ? pass16d_plan(pa, &mt, &nbt, true) : 0;
         int64_t unit = kPassRows;
         int tsm = 0;
         if (!red) {

@@ -250,9 +250,7 @@ hipError_t launch_wpass(int S, const PassArgs &a, int nwg, hipStream_t st);
 // Reduced-precision mixed form with double-buffered direct-to-LDS loads in 32-row tiles
 // (rows_per must be a multiple of 32): waves per workgroup (8 or 16), or 0
 // when it does not apply.
-// any_width: also below the column bound (reduced precisions, whose
-// 512-thread pass runs one workgroup per CU).  min_cols: the column bound
-// (0: the library's default).
+// any_width: every column count, else from min_cols columns on.
 int pass16d_plan(const PassArgs &a, int *mt, int *nb, bool any_width = false, int min_cols = 0);
 // Launch with the plan's waves per workgroup (nw) and N-tiles (nb): mx is
 // the reduced precision of the projection tiles from lpb on.
@@ -288,7 +286,6 @@ hipError_t launch_widen(const float *x, int64_t ldx, double *q, int64_t ldq, int
 // Zero n entries with a kernel (no memset nodes, so the sequence can be
 // captured in a graph).
 hipError_t launch_fill(double *p, size_t n, hipStream_t st);
-hipError_t launch_fill_int(int *p, size_t n, hipStream_t st);
 
 // Accuracy harness: Q^T Q with compensated (double-double) accumulation.
 // part receives, per row chunk (gram_dd_chunks(m) of them) and 64 x 64

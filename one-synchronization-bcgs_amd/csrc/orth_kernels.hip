@@ -528,11 +528,10 @@ hipError_t launch_widen(const float *x, int64_t ldx, double *q, int64_t ldq, int
     return hipGetLastError();
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_fill(T *p, size_t n)
+__global__ __launch_bounds__(256) void k_fill(double *p, size_t n)
 {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-        p[i] = T(0);
+        p[i] = 0.0;
 }
 
 hipError_t launch_fill(double *p, size_t n, hipStream_t st)
@@ -540,16 +539,7 @@ hipError_t launch_fill(double *p, size_t n, hipStream_t st)
     if (n == 0) return hipSuccess;
     size_t g = (n + 255) / 256;
     if (g > 4096) g = 4096;
-    k_fill<double><<<dim3((unsigned)g), dim3(256), 0, st>>>(p, n);
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_int(int *p, size_t n, hipStream_t st)
-{
-    if (n == 0) return hipSuccess;
-    size_t g = (n + 255) / 256;
-    if (g > 4096) g = 4096;
-    k_fill<int><<<dim3((unsigned)g), dim3(256), 0, st>>>(p, n);
+    k_fill<<<dim3((unsigned)g), dim3(256), 0, st>>>(p, n);
     return hipGetLastError();
 }
 

@@ -356,29 +356,23 @@ int pass16bm_plan(const PassArgs &a)
     return ts;
 }
 
-template <int MT, int NB, int F, bool EARLY, int MX>
-hipError_t launch_bm_t(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
-{
-    return launch_pass16b_v<MT, NB, F, EARLY, true, MX>(a, lds, nwg, st);
-}
-
 template <int MX>
 hipError_t launch_bm_mx(const PassArgs &a, int ts, int mt, int nb, size_t lds, int nwg,
                         hipStream_t st)
 {
     if (a.na == 0) {
         switch (ts) {
-        case 32: return launch_bm_t<1, 1, 1, true, MX>(a, lds, nwg, st);
-        case 64: return launch_bm_t<1, 1, 2, true, MX>(a, lds, nwg, st);
-        case 128: return launch_bm_t<1, 1, 4, true, MX>(a, lds, nwg, st);
-        case 256: return launch_bm_t<1, 1, 8, true, MX>(a, lds, nwg, st);
+        case 32: return launch_pass16b<1, 1, 1, true, MX>(a, lds, nwg, st);
+        case 64: return launch_pass16b<1, 1, 2, true, MX>(a, lds, nwg, st);
+        case 128: return launch_pass16b<1, 1, 4, true, MX>(a, lds, nwg, st);
+        case 256: return launch_pass16b<1, 1, 8, true, MX>(a, lds, nwg, st);
         default: return hipErrorInvalidValue;
         }
     }
 #define ORTH_BM(M, F)                                                                  \
     if (mt == M)                                                                       \
-        return nb == 2 ? launch_bm_t<M, 2, F, false, MX>(a, lds, nwg, st)              \
-                       : launch_bm_t<M, 1, F, false, MX>(a, lds, nwg, st);
+        return nb == 2 ? launch_pass16b<M, 2, F, false, MX>(a, lds, nwg, st)           \
+                       : launch_pass16b<M, 1, F, false, MX>(a, lds, nwg, st);
     switch (ts) {
     case 32:
         ORTH_BM(1, 1) ORTH_BM(2, 1) ORTH_BM(3, 1) ORTH_BM(4, 1)
@@ -412,18 +406,14 @@ hipError_t launch_pass16bm(const PassArgs &a, int mx, int nwg, hipStream_t st)
     }
 }
 
-// The double-buffered s = 16 pass (orth_pass16d.h) with 32-row tiles: waves
-// per workgroup (8: two workgroups per CU, when both buffers of two
-// workgroups fit a CU's LDS; 16: one workgroup per CU, up to the whole
-// 160 KB), or 0 when it does not apply.  It needs FP64 data with an even
-// row count and leading dimension and a 16-byte aligned slab (16-byte loads
-// of row pairs), the folded (non-sequential) step 1, and at least
-// kPass16dMinCols columns: measured at m = 2^24, n = 256, it beats k_pass16b
-// on the passes over 128 columns and more (by up to 0.8 ms each) and loses
-// on the narrower ones, where k_pass16b runs two workgroups per CU with 64-
-// to 256-row super-tiles (ORTH_PASS16D_MINCOLS overrides the bound).
-constexpr int kPass16dMinCols = 128;
-
+// The double-buffered pass (orth_pass16d.h) with 32-row tiles: waves per
+// workgroup (8: two workgroups per CU, when both buffers of two workgroups fit
+// a CU's LDS; 16: one workgroup per CU, up to the whole 160 KB), or 0 when it
+// does not apply.  It needs FP64 columns with an even row count and leading
+// dimension and a 16-byte aligned slab (16-byte loads of row pairs) and the
+// folded (non-sequential) step 1.  It takes every column count: the 512-thread
+// pass with super-tiles runs one workgroup per CU (ORTH_PASS16D_MINCOLS sets a
+// bound).
 int pass16d_plan(const PassArgs &a, int *mt, int *nb, bool any_width, int min_cols)
 {
     if (getenv("ORTH_PASS_REGPF")) return 0;
@@ -437,7 +427,7 @@ int pass16d_plan(const PassArgs &a, int *mt, int *nb, bool any_width, int min_co
     // Row pairs are loaded whole: an odd row count would read past the last
     // row of the last column.
     if (a.ldX % 2 != 0 || a.m % 2 != 0 || (uintptr_t)a.X % 16 != 0) return 0;
-    int minc = any_width ? 1 : min_cols > 0 ? min_cols : kPass16dMinCols;
+    int minc = any_width ? 1 : min_cols;
     if (const char *e = getenv("ORTH_PASS16D_MINCOLS")) minc = atoi(e);
     if (a.ncols < minc || a.ncols > a.wl) return 0;
     const bool force16 = getenv("ORTH_PASS16D_ONEWG") != nullptr;

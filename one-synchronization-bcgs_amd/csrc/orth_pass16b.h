@@ -1,8 +1,6 @@
-// The 512-thread fused pass for block width 16 (FP64 form and, through the
-// MX parameter, the mixed form), shared by the kernel translation units.
+// The 512-thread fused pass of the mixed form with reduced-precision products
+// (block width 16).
 #pragma once
-
-#include <type_traits>
 
 #include "orth_device.h"
 #include "orth_tail.h"
@@ -33,18 +31,17 @@ constexpr int kLpC = 5;
 
 // EARLY: passes without a projection issue the next tile's loads as soon as
 // the current tile is in LDS (nothing else would hide their latency).
-// V2: every thread loads two consecutive rows with one 16-byte load (needs
-// an even leading dimension and a 16-byte aligned slab).
-// MX (mixed form, kMx*; 0 = FP64 form): columns at or past raw0 come from
-// the FP32 input X32; when MX is a reduced precision, the products the host
-// marks (Z tiles consumed by lp groups, projection tiles whose B columns
+// Every thread loads two consecutive rows with one 16-byte load (needs an even
+// leading dimension and a 16-byte aligned slab).
+// MX (kMxBF16, kMxFP16, kMxBF16X3): columns at or past raw0 come from the
+// FP32 input X32; the products the host marks (Z tiles consumed by lp groups, projection tiles whose B columns
 // start at or past lpb) run on bf16 / fp16 MFMA with FP32 accumulation per
 // 32-row chunk, summed in FP64.
-template <int MT, int NB, int F, bool EARLY, bool V2, int MX = 0>
-// Reduced-precision forms run one workgroup per CU (their operand
-// conversions need more than the 128 registers of two).
-__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
-    MX != 0 ? 2 : 4, MX != 0 ? 2 : 4))) void k_pass16b(PassArgs a)
+// One workgroup per CU: the operand conversions need more than the 128
+// registers of two.
+template <int MT, int NB, int F, bool EARLY, int MX>
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_pass16b(
+    PassArgs a)
 {
     constexpr int N1 = 32, TS = 32 * F, LD = TS + 1;
     constexpr int LTS = F == 1 ? 5 : F == 2 ? 6 : F == 4 ? 7 : 8;
@@ -89,27 +86,25 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int j = 0; j < MT; j++) acc[j] = dbl4{0.0, 0.0, 0.0, 0.0};
 
-    // Mixed form: is this wave's Z tile (N-tile znt) a reduced-precision
+    // Is this wave's Z tile (N-tile znt) a reduced-precision
     // product, and its coefficient chunks [zq0, zq0 + zqn) as MFMA B
     // fragments (lane: k = 8 lk + e of column li), converted once.
-    constexpr bool LP = MX != 0;
-    constexpr int MXL = LP ? MX : kMxBF16;  // operand format of the reduced-precision paths
     const int znt = F == 1 ? (wave >> 1) & 1 : wave & 1;
-    const bool zlp = LP && !a.seq && ztile_lp(a, znt);
+    const bool zlp = !a.seq && ztile_lp(a, znt);
     int zq0 = 0, zqn = 0;
-    LpFrag<MXL> fbz[LP ? kLpC : 1];
-    if constexpr (LP) {
+    LpFrag<MX> fbz[kLpC];
+    {
         const int nch = (a.k1 + 31) >> 5;
         zq0 = F == 1 && (wave >> 2) ? nch >> 1 : 0;
         zqn = F == 1 ? ((wave >> 2) ? nch - (nch >> 1) : nch >> 1) : nch;
 #pragma unroll
         for (int c = 0; c < kLpC; c++) {
             const int k0 = 32 * (zq0 + c) + 8 * lk;
-            fbz[c] = lp_frag_g<MXL>(Cg + (int64_t)k0 * N1 + znt * 16 + li, N1,
+            fbz[c] = lp_frag_g<MX>(Cg + (int64_t)k0 * N1 + znt * 16 + li, N1,
                                    zlp && c < zqn ? a.k1 - k0 : 0);
         }
     }
-    const bool plp = LP && a.b0 + 16 * tb >= a.lpb;
+    const bool plp = a.b0 + 16 * tb >= a.lpb;
 
     const int64_t rb = (int64_t)blockIdx.x * a.rows_per;
     const int64_t re = min(a.m, rb + a.rows_per);
@@ -117,18 +112,15 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     constexpr int PSTEP = kB / TS;
     const int prow = tid & (TS - 1), pcol = tid >> LTS;
     // Loads: thread tid moves rows (2 (tid % (TS/2)), +1) of columns
-    // tid / (TS/2) + i (1024 / TS) when V2, else row tid % TS of columns
-    // tid / TS + i (512 / TS).
+    // tid / (TS/2) + i (1024 / TS).
     typedef double dbl2v __attribute__((ext_vector_type(2)));
-    constexpr int VR = V2 ? 2 : 1;               // rows per thread
-    constexpr int LSTEP = VR * kB / TS;          // columns per load step
-    constexpr int NPF = kBPF / VR;               // load steps
+    constexpr int VR = 2;                // rows per thread
+    constexpr int LSTEP = VR * kB / TS;  // columns per load step
+    constexpr int NPF = kBPF / VR;       // load steps
     const int lrow = VR * (tid & (TS / VR - 1)), lcol = tid / (TS / VR);
     const int lnld = (a.ncols - lcol + LSTEP - 1) / LSTEP;
-    const double *lx = a.X + lrow + (int64_t)lcol * a.ldX;
-    const int64_t lxs = (int64_t)LSTEP * a.ldX;
     const int lpl = lcol * LD + lrow;
-    typename std::conditional<V2, dbl2v, double>::type pf[NPF];
+    dbl2v pf[NPF];
     // Raw (FP32) columns: a.raw0 is a multiple of 16 and a wave's lanes move
     // at most four consecutive columns of a 4-aligned group, so whether load
     // step i is raw is uniform per wave.  A raw step moves RF = 2 VR FP32
@@ -141,84 +133,53 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     // addressed from a wave-uniform base (the wave's first load column) plus
     // one 32-bit byte offset per lane, below 16 ldX32 bytes (the host checks
     // the size and 16-byte alignment).
-    typedef float flt2v __attribute__((ext_vector_type(2)));
     typedef float flt4v __attribute__((ext_vector_type(4)));
     constexpr int RF = 2 * VR;
     const int lq = lrow / VR, rq = lq & (TS / RF - 1);
     const bool rstore = lq < TS / RF;
     auto raw_step = [&](int i) {
-        return MX != 0 && __builtin_amdgcn_readfirstlane((int)(lcol + i * LSTEP >= a.raw0)) != 0;
+        return __builtin_amdgcn_readfirstlane((int)(lcol + i * LSTEP >= a.raw0)) != 0;
     };
-    // The mixed form addresses its FP64 columns the same way, so a load step
-    // keeps no 64-bit lane address; row checks compare against the
-    // wave-uniform count of rows left in the super-tile.
-    const char *wx32 = nullptr, *wx64 = nullptr;
-    int64_t lxs32 = 0, lxs64 = 0;
-    uint32_t lb32 = 0, lb64 = 0;
-    if constexpr (MX != 0) {
-        const int wcol = __builtin_amdgcn_readfirstlane(lcol);
-        wx32 = (const char *)(a.X32 + (int64_t)wcol * a.ldX32);
-        wx64 = (const char *)(a.X + (int64_t)wcol * a.ldX);
-        lxs32 = (int64_t)LSTEP * a.ldX32 * 4;
-        lxs64 = (int64_t)LSTEP * a.ldX * 8;
-        lb32 = 4u * (uint32_t)(RF * rq + (lcol - wcol) * a.ldX32);
-        lb64 = 8u * (uint32_t)(lrow + (lcol - wcol) * a.ldX);
-    }
+    // The FP64 columns are addressed the same way, so a load step keeps no
+    // 64-bit lane address; row checks compare against the wave-uniform count
+    // of rows left in the super-tile.
+    const int wcol = __builtin_amdgcn_readfirstlane(lcol);
+    const char *wx32 = (const char *)(a.X32 + (int64_t)wcol * a.ldX32);
+    const char *wx64 = (const char *)(a.X + (int64_t)wcol * a.ldX);
+    const int64_t lxs32 = (int64_t)LSTEP * a.ldX32 * 4;
+    const int64_t lxs64 = (int64_t)LSTEP * a.ldX * 8;
+    const uint32_t lb32 = 4u * (uint32_t)(RF * rq + (lcol - wcol) * a.ldX32);
+    const uint32_t lb64 = 8u * (uint32_t)(lrow + (lcol - wcol) * a.ldX);
     auto load = [&](int64_t r0) {
-        if constexpr (MX != 0) {
-            const int rem = (int)min(re - r0, (int64_t)TS);
-            // The lane offsets are opaque to the optimizer here, so each
-            // address stays (uniform base) + (32-bit lane offset) instead of
-            // eight hoisted 64-bit lane addresses per source.
-            uint32_t o32 = lb32, o64 = lb64;
-            asm volatile("" : "+v"(o32), "+v"(o64));
-            const char *b32 = wx32 + 4 * r0, *b64 = wx64 + 8 * r0;
-            const bool ok1 = lrow < rem, ok2 = lrow + VR - 1 < rem, ok4 = RF * rq + RF - 1 < rem;
+        const int rem = (int)min(re - r0, (int64_t)TS);
+        // The lane offsets are opaque to the optimizer here, so each
+        // address stays (uniform base) + (32-bit lane offset) instead of
+        // eight hoisted 64-bit lane addresses per source.
+        uint32_t o32 = lb32, o64 = lb64;
+        asm volatile("" : "+v"(o32), "+v"(o64));
+        const char *b32 = wx32 + 4 * r0, *b64 = wx64 + 8 * r0;
+        const bool ok1 = lrow < rem, ok2 = lrow + VR - 1 < rem, ok4 = RF * rq + RF - 1 < rem;
 #pragma unroll
-            for (int i = 0; i < NPF; i++)
-                if (i < lnld) {
-                    using PV = typename std::remove_reference<decltype(pf[0])>::type;
-                    if (raw_step(i)) {
-                        const float *q32 = (const float *)(b32 + i * lxs32 + o32);
-                        if (ok4) {
-                            pf[i] = __builtin_nontemporal_load((const PV *)q32);
-                        } else {
-                            float v[RF];
-#pragma unroll
-                            for (int e = 0; e < RF; e++) v[e] = RF * rq + e < rem ? q32[e] : 0.f;
-                            if constexpr (V2)
-                                pf[i] = __builtin_bit_cast(dbl2v, flt4v{v[0], v[1], v[2], v[3]});
-                            else
-                                pf[i] = __builtin_bit_cast(double, flt2v{v[0], v[1]});
-                        }
+        for (int i = 0; i < NPF; i++)
+            if (i < lnld) {
+                if (raw_step(i)) {
+                    const float *q32 = (const float *)(b32 + i * lxs32 + o32);
+                    if (ok4) {
+                        pf[i] = __builtin_nontemporal_load((const dbl2v *)q32);
                     } else {
-                        const double *q64 = (const double *)(b64 + i * lxs64 + o64);
-                        if (ok2)
-                            pf[i] = __builtin_nontemporal_load((const PV *)q64);
-                        else if constexpr (V2)
-                            pf[i] = dbl2v{ok1 ? q64[0] : 0.0, 0.0};
-                        else
-                            pf[i] = 0.0;
+                        float v[RF];
+#pragma unroll
+                        for (int e = 0; e < RF; e++) v[e] = RF * rq + e < rem ? q32[e] : 0.f;
+                        pf[i] = __builtin_bit_cast(dbl2v, flt4v{v[0], v[1], v[2], v[3]});
                     }
-                }
-        } else if constexpr (V2) {
-            const double *q = lx + r0;
-            const bool ok2 = r0 + lrow + 1 < re, ok1 = r0 + lrow < re;
-#pragma unroll
-            for (int i = 0; i < NPF; i++)
-                if (i < lnld) {
+                } else {
+                    const double *q64 = (const double *)(b64 + i * lxs64 + o64);
                     if (ok2)
-                        pf[i] = __builtin_nontemporal_load((const dbl2v *)(q + i * lxs));
+                        pf[i] = __builtin_nontemporal_load((const dbl2v *)q64);
                     else
-                        pf[i] = dbl2v{ok1 ? q[i * lxs] : 0.0, 0.0};
+                        pf[i] = dbl2v{ok1 ? q64[0] : 0.0, 0.0};
                 }
-        } else {
-            const double *q = lx + r0;
-            const bool ok = r0 + lrow < re;
-#pragma unroll
-            for (int i = 0; i < NPF; i++)
-                if (i < lnld) pf[i] = ok ? __builtin_nontemporal_load(q + i * lxs) : 0.0;
-        }
+            }
     };
     if (rb < re) load(rb);
 
@@ -230,21 +191,13 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
                 if (raw_step(i)) {
                     if (rstore) {
                         double *d = sm + lcol * LD + RF * rq + i * LSTEP * LD;
-                        if constexpr (V2) {
-                            const flt4v v = __builtin_bit_cast(flt4v, pf[i]);
+                        const flt4v v = __builtin_bit_cast(flt4v, pf[i]);
 #pragma unroll
-                            for (int e = 0; e < 4; e++) d[e] = (double)v[e];
-                        } else {
-                            const flt2v v = __builtin_bit_cast(flt2v, pf[i]);
-                            d[0] = (double)v.x;
-                            d[1] = (double)v.y;
-                        }
+                        for (int e = 0; e < 4; e++) d[e] = (double)v[e];
                     }
-                } else if constexpr (V2) {
+                } else {
                     sm[lpl + i * LSTEP * LD] = pf[i].x;
                     sm[lpl + 1 + i * LSTEP * LD] = pf[i].y;
-                } else {
-                    sm[lpl + i * LSTEP * LD] = pf[i];
                 }
             }
         __syncthreads();
@@ -275,9 +228,9 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
                             for (int c = 0; c < kLpC; c++)
                                 if (c < zqn) {
                                     const int k0 = 32 * (zq0 + c) + 8 * lk;
-                                    const LpFrag<MXL> fa = lp_frag<MXL>(
+                                    const LpFrag<MX> fa = lp_frag<MX>(
                                         sm + min(k0, a.wl - 8) * LD + mt * 16 + li, LD);
-                                    t = lp_mma<MXL>(fa, fbz[c], t);
+                                    t = lp_mma<MX>(fa, fbz[c], t);
                                     __builtin_amdgcn_sched_barrier(0);
                                 }
                             z = dbl4{t[0], t[1], t[2], t[3]};
@@ -325,9 +278,9 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
                             for (int c = 0; c < kLpC; c++)
                                 if (c < zqn) {
                                     const int k0 = 32 * c + 8 * lk;
-                                    const LpFrag<MXL> fa = lp_frag<MXL>(
+                                    const LpFrag<MX> fa = lp_frag<MX>(
                                         sm + min(k0, a.wl - 8) * LD + (mt0 + 4 * j) * 16 + li, LD);
-                                    t = lp_mma<MXL>(fa, fbz[c], t);
+                                    t = lp_mma<MX>(fa, fbz[c], t);
                                     __builtin_amdgcn_sched_barrier(0);
                                 }
                             z[j] = dbl4{t[0], t[1], t[2], t[3]};
@@ -433,13 +386,13 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
             // accumulation within the chunk, FP64 across chunks.
 #pragma unroll 1
             for (int c = 0; c < F; c++) {
-                const LpFrag<MXL> fb =
-                    lp_frag<MXL>(sm + boff2 - lk + 32 * c + 8 * lk, 1);
+                const LpFrag<MX> fb =
+                    lp_frag<MX>(sm + boff2 - lk + 32 * c + 8 * lk, 1);
 #pragma unroll
                 for (int j = 0; j < MT; j++) {
-                    const LpFrag<MXL> fa =
-                        lp_frag<MXL>(sm + aoff2[j] - lk + 32 * c + 8 * lk, 1);
-                    const f32x4 t = lp_mma<MXL>(fa, fb, f32x4{0.f, 0.f, 0.f, 0.f});
+                    const LpFrag<MX> fa =
+                        lp_frag<MX>(sm + aoff2[j] - lk + 32 * c + 8 * lk, 1);
+                    const f32x4 t = lp_mma<MX>(fa, fb, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                     for (int v = 0; v < 4; v++) acc[j][v] += (double)t[v];
                     __builtin_amdgcn_sched_barrier(0);
@@ -456,9 +409,9 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
                 for (int j = 0; j < MT; j++)
                     acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[j], bc, acc[j], 0, 0, 0);
                 // Bound the operand loads in flight (register pressure): two
-                // k-steps, one in the mixed form's four-tile instances (their
-                // raw-column loader holds a few more registers).
-                if ((MX != 0 && MT >= 4) || (ks & 1) == 1) __builtin_amdgcn_sched_barrier(0);
+                // k-steps, one in the four-tile instances (their raw-column
+                // loader holds a few more registers).
+                if (MT >= 4 || (ks & 1) == 1) __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
@@ -481,20 +434,19 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     pass_tail(a, sm, kst, kB);
 }
 
-template <int MT, int NB, int F, bool EARLY, bool V2, int MX = 0>
-hipError_t launch_pass16b_v(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
+template <int MT, int NB, int F, bool EARLY, int MX>
+hipError_t launch_pass16b(const PassArgs &a, size_t lds, int nwg, hipStream_t st)
 {
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)k_pass16b<MT, NB, F, EARLY, V2, MX>,
+        hipError_t e = hipFuncSetAttribute((const void *)k_pass16b<MT, NB, F, EARLY, MX>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(160 * 1024));
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    k_pass16b<MT, NB, F, EARLY, V2, MX><<<dim3(nwg), dim3(kB), lds, st>>>(a);
+    k_pass16b<MT, NB, F, EARLY, MX><<<dim3(nwg), dim3(kB), lds, st>>>(a);
     return hipGetLastError();
 }
-
 
 }  // namespace orth

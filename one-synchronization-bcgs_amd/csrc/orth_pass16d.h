@@ -96,8 +96,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     PassArgs a)
 {
     constexpr int TS = 32, N1 = 32, kD = 64 * NW, LDc = kDLd;
-    constexpr bool MIX = MX != 0, LPP = MX != 0;
-    constexpr int MXL = LPP ? MX : kMxBF16;  // operand format of the reduced-precision products
     // Step-1 work items: 2 x 2 Z tiles of 16 x 16, the inner dimension
     // split KS ways so that the items fill the NW waves.
     constexpr int ZT = 4, KS = NW / ZT;
@@ -163,8 +161,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     // Reduced-precision N-tiles; their accumulators hold rows lk 4 + v.
     bool lowt[NB];
 #pragma unroll
-    for (int t = 0; t < NB; t++) lowt[t] = LPP && a.b0 + 16 * t >= a.lpb;
-    const bool anylow = LPP && lowt[NB - 1];
+    for (int t = 0; t < NB; t++) lowt[t] = a.b0 + 16 * t >= a.lpb;
+    const bool anylow = lowt[NB - 1];
     dbl4 acc[NB];
 #pragma unroll
     for (int t = 0; t < NB; t++) acc[t] = dbl4{0.0, 0.0, 0.0, 0.0};
@@ -176,8 +174,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const int64_t re = min(a.m, rb + a.rows_per);
     // Loads: slot span i (64 slots) goes to wave i % NW.  Slot q of column c
     // holds row pair q ^ 8 (c & 1) (the half swap); the pad slot repeats
-    // slot 15's row pair.  Mixed form: the DMA covers the columns below raw0.
-    const int ndma = MIX ? min(a.ncols, a.raw0) : a.ncols;
+    // slot 15's row pair.  The DMA covers the columns below raw0.
+    const int ndma = min(a.ncols, a.raw0);
     const int nspan = (ndma * kDSl + 63) / 64;
     const int64_t rlast = (a.m - 1) & ~(int64_t)1;  // last row-pair start
     // Spans of this wave: i = wave + NW j; those with j in [j0, j1) are
@@ -204,20 +202,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     // never used.
     typedef float flt4 __attribute__((ext_vector_type(4)));
     const int nraw = a.ncols - ndma;
-    const bool rv4 = MIX && a.ldX32 % 4 == 0 && (uintptr_t)a.X32 % 16 == 0;
+    const bool rv4 = a.ldX32 % 4 == 0 && (uintptr_t)a.X32 % 16 == 0;
     flt4 rv = flt4{0.f, 0.f, 0.f, 0.f};
     auto raw_issue = [&](int64_t r0) {
-        if constexpr (MIX) {
-            const int e = opaque(tid), c = e >> 3;
-            if (c < nraw) {
-                const int64_t row = r0 + 4 * (e & 7);
-                const float *p = a.X32 + (int64_t)(ndma + c) * a.ldX32;
-                if (rv4 && row + 3 < a.m) {
-                    rv = __builtin_nontemporal_load((const flt4 *)(p + row));
-                } else {
+        const int e = opaque(tid), c = e >> 3;
+        if (c < nraw) {
+            const int64_t row = r0 + 4 * (e & 7);
+            const float *p = a.X32 + (int64_t)(ndma + c) * a.ldX32;
+            if (rv4 && row + 3 < a.m) {
+                rv = __builtin_nontemporal_load((const flt4 *)(p + row));
+            } else {
 #pragma unroll
-                    for (int q = 0; q < 4; q++) rv[q] = __builtin_nontemporal_load(p + min(row + q, a.m - 1));
-                }
+                for (int q = 0; q < 4; q++) rv[q] = __builtin_nontemporal_load(p + min(row + q, a.m - 1));
             }
         }
     };
@@ -234,23 +230,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
         // makes all of them visible), and every wave is done with the other
         // buffer: stream tile i+1 into it.
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if constexpr (MIX) {
-            // This tile's raw columns, widened (rows past the slab: zero),
-            // before any load of the next tile is issued (a wait for the
-            // registers then waits for nothing in flight).
-            {
-                const int e = opaque(tid), c = e >> 3, r4 = 4 * (e & 7);
-                if (c < nraw) {
-                    double *d = cur + dpos(ndma + c, r4);
+        // This tile's raw columns, widened (rows past the slab: zero), before
+        // any load of the next tile is issued (a wait for the registers then
+        // waits for nothing in flight).
+        {
+            const int e = opaque(tid), c = e >> 3, r4 = 4 * (e & 7);
+            if (c < nraw) {
+                double *d = cur + dpos(ndma + c, r4);
 #pragma unroll
-                    for (int q = 0; q < 4; q++) d[q] = r0 + r4 + q < re ? (double)rv[q] : 0.0;
-                }
+                for (int q = 0; q < 4; q++) d[q] = r0 + r4 + q < re ? (double)rv[q] : 0.0;
             }
-            // With pending groups their solve, after two barriers, is the
-            // first reader of these columns; without, the projection reads
-            // them next.
-            if (nraw > 0 && a.ngrp == 0) lds_barrier();
         }
+        // With pending groups their solve, after two barriers, is the first
+        // reader of these columns; without, the projection reads them next.
+        if (nraw > 0 && a.ngrp == 0) lds_barrier();
         // The next tile's loads: by the waves that solve a group chunk in
         // this tile, and by all when no group is pending or no projection
         // follows the solve, at once; the other waves issue theirs while the
@@ -375,22 +368,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if constexpr (LPP) {
-            if (proj && anylow) {
-                // Operands: rows 8 lk .. 8 lk + 7 of column a0 + 16 w + li
-                // (A) and b0 + 16 t + li (B), eight consecutive doubles.
-                const LpFrag<MXL> fa =
-                    lp_frag<MXL>(cur + opaque(pab - lk + 8 * lk + (lk < 2 ? sa : -sa)), 1);
+        if (proj && anylow) {
+            // Operands: rows 8 lk .. 8 lk + 7 of column a0 + 16 w + li (A)
+            // and b0 + 16 t + li (B), eight consecutive doubles.
+            const LpFrag<MX> fa =
+                lp_frag<MX>(cur + opaque(pab - lk + 8 * lk + (lk < 2 ? sa : -sa)), 1);
 #pragma unroll
-                for (int t = 0; t < NB; t++)
-                    if (lowt[t]) {
-                        const LpFrag<MXL> fb = lp_frag<MXL>(
-                            cur + opaque(pbb - lk + 8 * lk + (lk < 2 ? sb : -sb)) + 16 * LDc * t, 1);
-                        const f32x4 tt = lp_mma<MXL>(fa, fb, f32x4{0.f, 0.f, 0.f, 0.f});
+            for (int t = 0; t < NB; t++)
+                if (lowt[t]) {
+                    const LpFrag<MX> fb = lp_frag<MX>(
+                        cur + opaque(pbb - lk + 8 * lk + (lk < 2 ? sb : -sb)) + 16 * LDc * t, 1);
+                    const f32x4 tt = lp_mma<MX>(fa, fb, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-                        for (int v = 0; v < 4; v++) acc[t][v] += (double)tt[v];
-                    }
-            }
+                    for (int v = 0; v < 4; v++) acc[t][v] += (double)tt[v];
+                }
         }
     }
 
