@@ -228,7 +228,7 @@ def suite(args):
               "cpu_rel_residual": inputs.rel_residual(Xh, Qo, Ro), "cpu_info_block": info[0]})
     del X0
 
-    # North-star shape, every variant, three conditionings; the mixed form
+    # The benchmark shape, every variant, three conditionings; the mixed form
     # (BCGSI+P-1S on the FP32-rounded input, four first-pass precisions)
     # beside FP64 BCGSI+P-1S on the same input, at four conditionings.
     m, n, s = 1 << 24, 256, 16

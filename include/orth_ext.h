@@ -108,11 +108,11 @@ int orth_bcgs_mixed_device(int variant, int precision, int64_t m, int64_t n,
  * device dR[i] (ld ldR[i]) receives R).  Instances run side by side on
  * several internal streams, each with private scratch; the batch is
  * captured into hipGraphs, at its second call in a row or after tuning, and
- * replayed while the same batch (shapes and pointers) is passed again.  tune != 0 first times the stream count and
- * workgroup share on this batch and keeps the best for batches with the
- * same shapes; it also decides between replaying captured graphs and
- * launching directly on the streams, and picks the tile shape of the s = 16
- * passes.  When the environment variable ORTH_TUNE_CACHE names a file, the
+ * replayed while the same batch (shapes and pointers) is passed again.
+ * tune != 0 first times the stream count and workgroup share on this batch
+ * and keeps the best for batches with the same shapes; it also decides
+ * between replaying captured graphs and launching directly on the streams.
+ * When the environment variable ORTH_TUNE_CACHE names a file, the
  * tuned configurations are written there (one text line per device and
  * batch shape) and read back by later processes, so that a call with
  * tune == 0 uses a stored configuration.  Batches larger than a graph-size

@@ -1404,11 +1404,11 @@ bool batch_capture(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg)
 // first time is launched directly on the streams (which also makes every
 // kernel's first launch, and its launch attributes, happen outside capture).
 // When the next call is for the same batch, it is captured and the graphs are
-// replayed at once; with `capture` the first run is followed by the capture.
-// Not every first run: a caller with new buffers in every call would pay for
-// graphs it never replays.  48 uneven instances of 2^12 to 2^18 rows: first
-// call 12.7 ms, second 11.0 (13.8 as a direct run followed by the capture),
-// the others 8.7.
+// replayed at once; with `capture` (the tuner) the first run is followed by
+// the capture.  Not every first run: a caller with new buffers in every call
+// would pay for graphs it never replays.  48 uneven instances of 2^12 to 2^18
+// rows: first call 12.7 ms, second 11.0 (13.8 as a direct run followed by the
+// capture), the others 8.7.
 bool batch_run(BatchCtx &b, const BatchArgs &a, const BatchCfg &cfg, bool capture)
 {
     const std::vector<int64_t> key = full_key(a, cfg);

@@ -17,9 +17,12 @@
 // the only vector-memory wait is the one that opens a tile.
 //
 // LDS layout of a buffer (see tpos): column c at c * TS doubles, its 16-byte
-// slots (row pairs) permuted by XOR with swz(c), so that both operand reads
-// spread over all 64 banks: 16 columns x 2 rows (projection) and 16 rows x 2
-// columns (step 1).  No padding: a load instruction moves 64 slots of data.
+// slots (row pairs) permuted by XOR with swz(c), so that an operand read by
+// itself spreads over all 64 banks: 16 columns x 2 rows (projection) and 16
+// rows x 2 columns (step 1).  Measured in conflict cycles per LDS cycle: none
+// in 16-row tiles with one N-tile, 0 to 14 % in 128-row ones, 23 to 39 % with
+// two N-tiles, whose operands sit on the same banks as each other.  No
+// padding: a load instruction moves 64 slots of data.
 //
 // Per tile: step 1 (Z = tile(:, 0:k1) C, 16 x 16 tiles of Z over the waves,
 // the inner dimension split KS ways when there are fewer tiles than waves);

@@ -20,8 +20,8 @@
 // part of the projection that no group takes part in.  Z and the solve are
 // transposed, as in the tile pass.
 //
-// 2^22 x 512, s = 32, P-1S: 110 ms (F = 4 m n^2 at 40 TFLOP/s) where separate
-// projection and update kernels took 178.
+// 2^22 x 512, s = 32, P-1S: 112 ms, 110 of them in 20 passes (F = 4 m n^2 at
+// 39 TFLOP/s), where separate projection and update kernels took 178.
 #pragma once
 
 #include "orth_tpass.h"
