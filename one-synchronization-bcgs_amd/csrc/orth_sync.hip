@@ -14,25 +14,25 @@
 
 namespace orth {
 
-// Sums of the partials of 32 elements in the fixed order of the in-pass tail
-// (tail_group), by NT threads: thread (el, q) sums groups q, q + NT / 32, ...
-// of element blockIdx.x * 32 + el into red, then q == 0 adds the group sums in
+// Sums of the partials of EL elements in the fixed order of the in-pass tail
+// (tail_group), by NT threads: thread (el, q) sums groups q, q + NT / EL, ...
+// of element blockIdx.x * EL + el into red, then q == 0 adds the group sums in
 // order.
-template <int NT>
+template <int NT, int EL = 32>
 static __device__ __forceinline__ double reduce_fixed_order(const double *__restrict__ part, int nwg,
                                                             int grp, int64_t E, double *red)
 {
-    const int el = threadIdx.x & 31, q = threadIdx.x >> 5;
-    const int64_t e = (int64_t)blockIdx.x * 32 + el;
+    const int el = threadIdx.x % EL, q = threadIdx.x / EL;
+    const int64_t e = (int64_t)blockIdx.x * EL + el;
     const int ngrp = (nwg + grp - 1) / grp;
     if (e < E)
-        for (int g = q; g < ngrp; g += NT / 32)
-            red[32 * g + el] = part_range_sum(part, E, e, g * grp, min(nwg, g * grp + grp));
+        for (int g = q; g < ngrp; g += NT / EL)
+            red[EL * g + el] = part_range_sum(part, E, e, g * grp, min(nwg, g * grp + grp));
     __syncthreads();
     double t = 0.0;
     if (q == 0 && e < E) {
         t = red[el];
-        for (int g = 1; g < ngrp; g++) t += red[32 * g + el];
+        for (int g = 1; g < ngrp; g++) t += red[EL * g + el];
     }
     return t;
 }
@@ -64,24 +64,34 @@ hipError_t launch_reduce(const double *part, int nwg, int64_t na, int64_t nb, do
 static int small_width(const SmallArgs &a) { return a.S <= 16 ? 16 : 32; }
 
 // k_reduce's fixed-order sum, then the small step in the last workgroup to
-// finish (ticket counter, publication as in the in-pass tail).  1024 threads:
-// a thread sums one group of partials (one memory round trip), and the small
-// step has 16 waves for its prefix Gram and its rows of R and C.
+// finish (ticket counter, publication as in the in-pass tail).  32 threads for
+// each of EL elements: a thread sums one group of partials (one memory round
+// trip).  With 1024 threads the small step has 16 waves for its prefix Gram and
+// its rows of R and C.
 constexpr int kRS = 1024;
-template <int W>
-__global__ __launch_bounds__(kRS) void k_reduce_small(const double *__restrict__ part, int nwg,
-                                                      int grp, int64_t E, double *out,
-                                                      int *ticket, SmallArgs sm)
+template <int W, int NT, int EL>
+__global__ __launch_bounds__(NT) void k_reduce_small(const double *__restrict__ part, int nwg,
+                                                     int grp, int64_t E, double *out,
+                                                     int *ticket, SmallArgs sm)
 {
-    constexpr int N = small_lds<W>() > kTailMaxGroups * 32 ? small_lds<W>() : kTailMaxGroups * 32;
+    constexpr int N = small_lds<W>() > kTailMaxGroups * EL ? small_lds<W>() : kTailMaxGroups * EL;
     __shared__ double lds[N];
     __shared__ int last;
-    const double t = reduce_fixed_order<kRS>(part, nwg, grp, E, lds);
-    const int64_t e = (int64_t)blockIdx.x * 32 + (threadIdx.x & 31);
-    if ((threadIdx.x >> 5) == 0 && e < E) out[e] = t;
+    const double t = reduce_fixed_order<NT, EL>(part, nwg, grp, E, lds);
+    const int64_t e = (int64_t)blockIdx.x * EL + threadIdx.x % EL;
+    if (threadIdx.x / EL == 0 && e < E) out[e] = t;
     if (!tail_ticket(ticket, (int)gridDim.x - 1, &last)) return;
     if (threadIdx.x == 0) *ticket = 0;
-    small_step<W>(kRS, sm, lds);
+    small_step<W>(NT, sm, lds);
+}
+
+template <int W, int NT, int EL>
+static hipError_t launch_rs(const double *part, int nwg, int64_t E, double *out, int *ticket,
+                            const SmallArgs &sm, hipStream_t st)
+{
+    k_reduce_small<W, NT, EL><<<dim3((unsigned)((E + EL - 1) / EL)), dim3(NT), 0, st>>>(
+        part, nwg, tail_group(nwg), E, out, ticket, sm);
+    return hipGetLastError();
 }
 
 hipError_t launch_reduce_small(const double *part, int nwg, int64_t na, int64_t nb, double *out,
@@ -89,12 +99,15 @@ hipError_t launch_reduce_small(const double *part, int nwg, int64_t na, int64_t 
 {
     const int64_t E = na * nb;
     if (E <= 0) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((E + 31) / 32)), block(kRS);
-    if (small_width(sm) == 16)
-        k_reduce_small<16><<<grid, block, 0, st>>>(part, nwg, tail_group(nwg), E, out, ticket, sm);
-    else
-        k_reduce_small<32><<<grid, block, 0, st>>>(part, nwg, tail_group(nwg), E, out, ticket, sm);
-    return hipGetLastError();
+    // A CholQR step has no prefix, so 16 waves of it only wait at each other's
+    // barriers: 256 threads, 8 elements each workgroup, up to 128 elements
+    // (blocks of 11).  BCGSI+ with 1024 / 256 threads, 4099 rows: 64 x 2 3.93 /
+    // 3.60 ms, 64 x 4 2.04 / 1.90, 200 x 10 3.08 / 3.00; 256 x 16 even (2.90 /
+    // 2.86, P-2S 1.83 / 1.84), 96 x 24 0.94 / 1.07.
+    if (small_width(sm) > 16) return launch_rs<32, kRS, 32>(part, nwg, E, out, ticket, sm, st);
+    return sm.op >= OP_CQR1 && sm.op <= OP_CQR3 && E <= 128
+               ? launch_rs<16, 256, 8>(part, nwg, E, out, ticket, sm, st)
+               : launch_rs<16, kRS, 32>(part, nwg, E, out, ticket, sm, st);
 }
 
 // ---------------------------------------------------------------------------
